@@ -83,6 +83,8 @@ SIGNATURES: dict[str, list] = {
     "axk_paged_kv_write_i8": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _vp],
     "axk_paged_decode_i8": [_vp] * 7 + [_i64] * 6 + [ctypes.c_float, _vp, ctypes.c_size_t, _vp],
     "axk_paged_prefill": [_vp] * 7 + [_i64] * 7 + [ctypes.c_float, _vp, _vp],
+    "axk_paged_prefill_workspace_size": [_i64] * 5,
+    "axk_paged_prefill_split": [_vp] * 7 + [_i64] * 7 + [ctypes.c_float, _vp, _vp, ctypes.c_size_t, _vp],
     "axk_gdn_recurrent": [_vp] * 10 + [_i64] * 6 + [_vp],
     "axk_gdn_chunk_workspace_size": [_i64] * 7,
     "axk_gdn_chunk_prefill": [_vp] * 10 + [_i64] * 7 + [_vp, ctypes.c_size_t, _vp],
@@ -133,6 +135,7 @@ _RESTYPES = {
     "axk_version": ctypes.c_char_p,
     "axk_status_string": ctypes.c_char_p,
     "axk_paged_decode_workspace_size": ctypes.c_size_t,
+    "axk_paged_prefill_workspace_size": ctypes.c_size_t,
     "axk_moe_workspace_size": ctypes.c_size_t,
     "axk_gdn_chunk_workspace_size": ctypes.c_size_t,
     "axk_gdn_layer_workspace_size": ctypes.c_size_t,

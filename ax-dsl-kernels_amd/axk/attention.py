@@ -332,9 +332,19 @@ def paged_prefill(
         _check(status.dtype == torch.int32 and status.numel() >= 1, "status must be int32 [1]")
         tensors.append(status)
     _lib.require_device(*tensors)
-    _lib.call(
-        "axk_paged_prefill", q.data_ptr(), kv_cache.data_ptr(), qo_indptr.data_ptr(), indptr.data_ptr(),
-        indices.data_ptr(), last_page_len.data_ptr(), output.data_ptr(), b, t, hq, hkv, d, page, p, float(sm_scale),
-        _lib.ptr(status), _lib.stream_of(q),
-    )
+    args = (q.data_ptr(), kv_cache.data_ptr(), qo_indptr.data_ptr(), indptr.data_ptr(), indices.data_ptr(),
+            last_page_len.data_ptr(), output.data_ptr(), b, t, hq, hkv, d, page, p, float(sm_scale),
+            _lib.ptr(status))
+    # few row blocks over a long history: the cached tokens are split over more workgroups (fp32 partials in a scratch
+    # tensor). Up to 320 cached tokens (the page table bounds them) a split is one or two pieces of 256 and its merge
+    # launch costs more than it gives (32 new tokens, HQ 16, HKV 2, D 256: at 232 cached tokens 20.9 us unsplit, 23.5
+    # split).
+    scratch = 0
+    if indices.numel() * page > 320:
+        scratch = _lib.load().axk_paged_prefill_workspace_size(b, t, hq, hkv, d)
+    if scratch:
+        ws = torch.empty(scratch, dtype=torch.uint8, device=q.device)
+        _lib.call("axk_paged_prefill_split", *args, ws.data_ptr(), scratch, _lib.stream_of(q))
+    else:
+        _lib.call("axk_paged_prefill", *args, _lib.stream_of(q))
     return output

@@ -201,6 +201,21 @@ AXK_DEV void lds_dma16_so(const void* sbase_any, uint32_t voff, uint32_t lds_bas
       : "memory");
 }
 
+// ... and with the default policy, for tiles other workgroups re-read through L2. `sbase` must be in scalar
+// registers already (uniform_ptr); the bytes land at lds_base + OFF + 16 * lane. M0 is not kept (nothing else here uses it);
+// the wait state after its write is the one LDS DMA needs.
+template <int OFF>
+AXK_DEV void lds_dma16_su_cached(const void* sbase, uint32_t voff, uint32_t lds_base_any) {
+  const uint32_t lds_base = __builtin_amdgcn_readfirstlane(lds_base_any);
+  asm volatile(
+      "s_add_u32 m0, %0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, %3"
+      :
+      : "s"(lds_base), "n"(OFF), "v"(voff), "s"(sbase)
+      : "memory", "scc");
+}
+
 template <int N>
 AXK_DEV void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

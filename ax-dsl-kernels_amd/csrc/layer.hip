@@ -469,13 +469,16 @@ int check_prefill(int64_t B, int64_t T, int64_t H, int64_t F) {
   return AXK_OK;
 }
 
+// With `splits`, the attention's KV-split scratch follows the buffers the layer cannot do without: the size queries
+// include it, while a call is accepted without it (the attention then runs unsplit).
 size_t attn_rows_ws(int64_t B, int64_t T, int64_t H, int64_t HQ, int64_t HKV, int64_t D, int64_t F,
-                    const axk_moe_block* moe = nullptr) {
+                    const axk_moe_block* moe = nullptr, bool splits = false) {
   if (HQ <= 0 || HKV <= 0 || HQ % HKV != 0 || !(D == 64 || D == 128 || D == 256)) return 0;
   if (moe && moe_ws_bytes(B * T, H, *moe) == 0) return 0;
   Carver c{nullptr};
   carve_attn_verify(c, B, B * T, H, HQ, HKV, D, F);
   if (moe) carve_moe(c, B * T, H, *moe);
+  if (splits) c.take<unsigned char>(axk_paged_prefill_workspace_size(B, B * T, HQ, HKV, D));
   return c.off;
 }
 
@@ -504,6 +507,8 @@ int attn_rows_impl(const uint16_t* x, const float* ln1, const uint8_t* w_q, cons
   Carver c{static_cast<unsigned char*>(workspace)};
   const AttnVerifyBufs a = carve_attn_verify(c, B, R, H, HQ, HKV, D, F);
   const MoeBufs eb = moe ? carve_moe(c, R, H, *moe) : MoeBufs{};
+  unsigned char* split_ws = workspace_bytes > c.off ? c.base + c.off : nullptr;
+  const size_t split_bytes = split_ws ? workspace_bytes - c.off : 0;
   const MlpWeights mw{mlp_gate_w, mlp_up_w, mlp_down_w, mlp_gate_s, mlp_up_s, mlp_down_s};
   auto body = [&]() -> int {
     AXK_TRY(axk_rmsnorm(x, H, ln1, a.h, H, R, H, eps, stream));
@@ -515,7 +520,8 @@ int attn_rows_impl(const uint16_t* x, const float* ln1, const uint8_t* w_q, cons
     AXK_TRY(axk_fill_iota_i32(a.qo_indptr, B, T, axk_stream(stream)));
     // the attention with its output gate applied as each row is written: gated = bf16(attn * sigmoid(gate))
     AXK_TRY(axk_paged_prefill_gated(a.q, kv_cache, a.qo_indptr, indptr, indices, last_page_len, a.qg + D, 2 * D,
-                                    a.gated, B, R, HQ, HKV, D, page_size, num_pages, sm_scale, axk_stream(stream)));
+                                    a.gated, B, R, HQ, HKV, D, page_size, num_pages, sm_scale, split_ws, split_bytes,
+                                    axk_stream(stream)));
     const AxkMxMat o = proj_mat(proj_fmt, w_o, s_o, a.y, H);
     AXK_TRY(projs(proj_fmt, a.gated, HQ * D, &o, 1, R, HQ * D, stream));
     if (moe) return moe_residual(x, a.y, ln2, mw, mlp_fmt, *moe, out, a.mlp, eb, R, H, F, eps, stream);
@@ -599,7 +605,7 @@ extern "C" size_t axk_attn_layer_verify_workspace_size(int64_t batch, int64_t to
                                                        int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
                                                        int64_t inter) {
   if (check_verify(batch, tokens, hidden, inter) != AXK_OK) return 0;
-  return attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter);
+  return attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter, nullptr, true);
 }
 
 extern "C" int axk_attn_layer_verify(
@@ -612,8 +618,8 @@ extern "C" int axk_attn_layer_verify(
     int64_t tokens, int64_t hidden, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t rot,
     int64_t page_size, int64_t num_pages, int64_t inter, float eps, float sm_scale, int proj_fmt, int mlp_fmt,
     void* workspace, size_t workspace_bytes, axk_stream_t stream) {
-  const size_t need = axk_attn_layer_verify_workspace_size(batch, tokens, hidden, num_qo_heads, num_kv_heads,
-                                                           head_dim, inter);
+  const size_t need = check_verify(batch, tokens, hidden, inter) == AXK_OK
+                          ? attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter) : 0;
   return attn_rows_impl(x, ln1, w_q, s_q, w_k, s_k, w_v, s_v, q_norm, k_norm, cos, sin, kv_cache, indptr, indices,
                         last_page_len, cache_location, w_o, s_o, ln2, mlp_gate_w, mlp_gate_s, mlp_up_w, mlp_up_s,
                         mlp_down_w, mlp_down_s, nullptr, out, batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, rot,
@@ -772,7 +778,7 @@ extern "C" size_t axk_attn_layer_prefill_workspace_size(int64_t batch, int64_t t
                                                         int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
                                                         int64_t inter) {
   if (check_prefill(batch, tokens, hidden, inter) != AXK_OK) return 0;
-  return attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter);
+  return attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter, nullptr, true);
 }
 
 extern "C" size_t axk_attn_layer_prefill_moe_workspace_size(int64_t batch, int64_t tokens, int64_t hidden,
@@ -780,7 +786,7 @@ extern "C" size_t axk_attn_layer_prefill_moe_workspace_size(int64_t batch, int64
                                                             int64_t head_dim, int64_t inter,
                                                             const axk_moe_block* moe) {
   if (!moe || check_prefill(batch, tokens, hidden, inter) != AXK_OK) return 0;
-  return attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter, moe);
+  return attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter, moe, true);
 }
 
 extern "C" int axk_attn_layer_prefill(
@@ -793,8 +799,8 @@ extern "C" int axk_attn_layer_prefill(
     int64_t tokens, int64_t hidden, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t rot,
     int64_t page_size, int64_t num_pages, int64_t inter, float eps, float sm_scale, int proj_fmt, int mlp_fmt,
     void* workspace, size_t workspace_bytes, axk_stream_t stream) {
-  const size_t need = axk_attn_layer_prefill_workspace_size(batch, tokens, hidden, num_qo_heads, num_kv_heads,
-                                                            head_dim, inter);
+  const size_t need = check_prefill(batch, tokens, hidden, inter) == AXK_OK
+                          ? attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter) : 0;
   return attn_rows_impl(x, ln1, w_q, s_q, w_k, s_k, w_v, s_v, q_norm, k_norm, cos, sin, kv_cache, indptr, indices,
                         last_page_len, cache_location, w_o, s_o, ln2, mlp_gate_w, mlp_gate_s, mlp_up_w, mlp_up_s,
                         mlp_down_w, mlp_down_s, nullptr, out, batch, tokens, hidden, num_qo_heads, num_kv_heads,
@@ -813,8 +819,8 @@ extern "C" int axk_attn_layer_prefill_moe(
     int64_t head_dim, int64_t rot, int64_t page_size, int64_t num_pages, int64_t inter, float eps, float sm_scale,
     int proj_fmt, int mlp_fmt, void* workspace, size_t workspace_bytes, axk_stream_t stream) {
   AXK_REQUIRE(moe, AXK_E_NULL);
-  const size_t need = axk_attn_layer_prefill_moe_workspace_size(batch, tokens, hidden, num_qo_heads, num_kv_heads,
-                                                                head_dim, inter, moe);
+  const size_t need = check_prefill(batch, tokens, hidden, inter) == AXK_OK
+                          ? attn_rows_ws(batch, tokens, hidden, num_qo_heads, num_kv_heads, head_dim, inter, moe) : 0;
   return attn_rows_impl(x, ln1, w_q, s_q, w_k, s_k, w_v, s_v, q_norm, k_norm, cos, sin, kv_cache, indptr, indices,
                         last_page_len, cache_location, w_o, s_o, ln2, mlp_gate_w, mlp_gate_s, mlp_up_w, mlp_up_s,
                         mlp_down_w, mlp_down_s, moe, out, batch, tokens, hidden, num_qo_heads, num_kv_heads,

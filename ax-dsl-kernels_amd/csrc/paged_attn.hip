@@ -24,7 +24,10 @@
 //              output for sequences without pages. A separate launch on purpose: merging inside the
 //              decode kernel needs a device-scope release/acquire per workgroup, which on a multi-XCD
 //              part writes back and invalidates the whole L2 and serialises the kernel.
+#include <algorithm>
 #include <mutex>
+#include <type_traits>
+#include <utility>
 
 #include "axk_common.h"
 #include "axk_host.h"
@@ -37,6 +40,7 @@ constexpr int kNBufPair = 4;  // bf16 LDS ring: two tile pairs, one landing whil
 constexpr int kTargetItems = 1024;
 constexpr int kMaxGroup = 16;  // query heads per KV head (MFMA N tile)
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kPfSlots = 256;  // workgroups of the prefill kernel that a split aims at
 
 struct PlanHeader {
   int n_items;
@@ -1126,46 +1130,81 @@ __global__ __launch_bounds__(256) void paged_kv_write_fp8_kernel(const uint16_t*
 // so token t sits at position kv_len - qlen + t and sees cached tokens 0 .. that position (the causal bias of the
 // current block, flash_attn.py:484-486; q35_prefill.py:264-300 masks the block the same way). The query rows of one
 // (sequence, KV head) are r = t * G + h for the G query heads h of the KV head: a workgroup takes 128 consecutive
-// rows (8 waves x 16) and streams the K / V tiles its rows can see, up to its last row's position, through a
-// direct-to-LDS ring (the decode kernel's tile layout, loads issued by the first 4 waves). Each wave computes
-// S^T = K Q^T for its 16 rows and O^T += V^T P^T over the whole head dim. 16 rows per wave keep Q and O in
-// 100 VGPRs (two waves per SIMD); 32 rows per wave overflowed the VGPRs and the compiler moved O between AGPRs and
-// VGPRs on every tile (measured: 700 VALU instructions per tile, 608 us for the 4096-token chunk).
+// rows (4 waves x 32) and streams the K / V tiles its rows can see, up to its last row's position, 32 tokens (a pair
+// of 16-token tiles) at a time through a direct-to-LDS ring.
+//
+// Each wave computes S^T = K Q^T (32 tokens x its 32 rows, 32x32x16 MFMA) and O^T += V^T P^T over the whole head dim:
+// 32 rows a wave, since every K / V byte read from LDS then feeds twice the MFMA work of 16 rows, and one row's 32
+// scores sit in two lanes (a single cross-lane step per maximum, none per sum). Q (64 VGPRs at D = 256) and O (128)
+// take most of a wave's registers, so at D = 256 a SIMD has one wave (two waves a SIMD spill 22 registers and, with
+// half the ring each, took 397 us where this takes 178). The score accumulator is the P^T operand as it stands: MFMA
+// k index (half h, j) is token 8 (j / 4) + 4 h + j % 4 of its 16-token tile, and V^T is read (transposing LDS reads)
+// in that order.
+//
+// What bounds it: one wave issues at most one instruction every four cycles, and a pair's 32 MFMAs (1024 cycles)
+// bring about 300 others. Measured at D = 256, HQ 16, HKV 2: a 4096-token chunk 178 us, 773 TFLOP/s (237 us with 16
+// rows a wave, 16x16x32 MFMA and two waves a SIMD); 256 tokens after 16000 cached ones 96 us with the KV splits
+// (814 us before: 32 row blocks on 256 CUs).
 typedef short axk_s16x8 __attribute__((ext_vector_type(8)));
-constexpr int kPfWaves = 8;
-constexpr int kPfRowsPerWave = 16;
-constexpr int kPfNI = kPfRowsPerWave / 16;  // 16-row MFMA blocks per wave
-constexpr int kPfRows = kPfWaves * kPfRowsPerWave;
-constexpr int kPfAhead = 6;  // tiles in flight while two are computed (even: tiles are taken in pairs)
-constexpr int kPfBuf = kPfAhead + 2;
+typedef float axk_f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kPfWaves = 4;
+constexpr int kPfRows = 32 * kPfWaves;
+constexpr int kPfRing = 4;       // tile pairs in the LDS ring
+constexpr int kPfMinPairs = 8;   // a split's shortest piece (256 tokens)
+constexpr int kPfMaxSplits = 64;
+constexpr int kPfMergeRows = 8;  // rows of one merge workgroup
 
+// The LDS image of a 16-token tile: K rows then V rows, no padding. Chunk c (16 bytes) of K row r is kept at chunk
+// c ^ (r mod 16) and of V row r at c ^ 4 (r mod 4), so that a K fragment read (16 rows, one chunk each) and a
+// transposing V read (4 rows, 64 bytes each) both cover all LDS banks.
 template <int D>
-__global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_kernel(
-    const uint16_t* __restrict__ q, const unsigned char* __restrict__ cache, const int* __restrict__ qo_indptr,
-    const int* __restrict__ indptr, const int* __restrict__ last_page_len, const int* __restrict__ indices,
-    int batch, int total_q, int hq, int hkv, int page_size, int64_t num_pages, float sm_scale, int xcd_per_head,
-    int* __restrict__ status, uint16_t* __restrict__ out, const uint16_t* __restrict__ gate, int64_t ldg) {
-  using C = PagedCfg<D>;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int group = hq / hkv;
-  // KV head and block index: consecutive workgroups go to the 8 XCDs in turn, so with xcd_per_head > 0 the blocks of
-  // one KV head run on xcd_per_head XCDs only and its K / V stay in their L2s
-  int kvh, want;
-  if (xcd_per_head > 0) {
-    const int x = blockIdx.x & 7, sl = blockIdx.x >> 3;
-    kvh = x / xcd_per_head;
-    want = sl * xcd_per_head + (x - kvh * xcd_per_head);
-  } else {
-    kvh = blockIdx.x % hkv;
-    want = blockIdx.x / hkv;
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int l16 = lane & 15, g = lane >> 4;
+struct PfCfg {
+  static constexpr int KS = D / 16;            // 16-deep MFMA steps of Q K^T
+  static constexpr int DT = D / 32;            // 32-wide tiles of O
+  static constexpr int RB = D * 2;             // bytes per cached row of one KV head
+  static constexpr int NCH = RB / 16;          // 16-byte chunks per row
+  static constexpr int RPI = 1024 / RB;        // rows per direct-to-LDS instruction (64 lanes x 16 B)
+  static constexpr int IPP = kTile / RPI;      // instructions per plane (K or V) of a tile
+  static constexpr int IPW = 2 * IPP / kPfWaves;  // instructions per wave per tile
+  static constexpr int PLANE = kTile * RB;
+  static constexpr int BUF = 2 * PLANE;        // one tile
+  static constexpr int PAIR = 2 * BUF;
+  static_assert(IPW >= 1 && IPW * kPfWaves == 2 * IPP && IPP % IPW == 0, "each wave loads rows of one plane");
+  static AXK_DEV int kswz(int r) { return r & (NCH < 16 ? NCH - 1 : 15); }
+  static AXK_DEV int vswz(int r) { return NCH < 16 ? ((r >> 1) & 1) : (r & 3); }  // in units of 4 chunks
+};
 
-  // this workgroup's (sequence, row block): the blocks of each sequence in turn, its last (longest) block first.
-  // Every wave derives the same answer; the grid is an upper bound and surplus workgroups return.
-  int b = -1, blk = 0;
-  for (int c0 = 0, base = 0; c0 < batch && b < 0; c0 += 64) {
+AXK_DEV axk_f32x16 mfma_bf16_32x32x16(axk_bf16x8 a, axk_bf16x8 b, axk_f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// f(std::integral_constant<int, 0>) .. f(<N - 1>): an unrolled loop whose index is a constant expression.
+template <typename F, int... I>
+AXK_DEV void for_each_index_of(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+AXK_DEV void for_each_index(F& f) {
+  for_each_index_of(f, std::make_integer_sequence<int, N>{});
+}
+
+// Row block `want` of one KV head: the blocks of each sequence in turn, its last (longest) block first. Every wave
+// derives the same answer; the grid is an upper bound and surplus workgroups get b = -1.
+struct PfBlock {
+  int b, r_first, r_last, q0, qlen;
+  int pb, npg, last, kv_len;    // page range, valid tokens of the last page, cached tokens
+  int base_pos;                 // position of new token 0
+  int ntiles;                   // tiles up to the block's last row's position
+  int piece, ns;                // pairs per split of the sequence, splits this block has
+};
+
+AXK_DEV PfBlock pf_block(int want, const int* __restrict__ qo_indptr, const int* __restrict__ indptr,
+                         const int* __restrict__ last_page_len, int batch, int group, int page_size, int nsplit) {
+  const int lane = threadIdx.x & 63;
+  PfBlock k;
+  k.b = -1;
+  int blk = 0;
+  for (int c0 = 0, base = 0; c0 < batch && k.b < 0; c0 += 64) {
     const int sq = c0 + lane;
     const int qlen_l = sq < batch ? qo_indptr[sq + 1] - qo_indptr[sq] : 0;
     const int nb = qlen_l > 0 ? (qlen_l * group + kPfRows - 1) / kPfRows : 0;
@@ -1179,257 +1218,516 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_kernel(
     const unsigned long long hit = __builtin_amdgcn_ballot_w64(nb > 0 && want >= excl && want < excl + nb);
     if (hit) {
       const int hl = __builtin_ctzll(hit);
-      b = c0 + hl;
+      k.b = c0 + hl;
       blk = __shfl(nb, hl, 64) - 1 - (want - __shfl(excl, hl, 64));
     }
     base += __shfl(incl, 63, 64);
   }
-  if (b < 0) return;
-  const int q0 = qo_indptr[b], qlen = qo_indptr[b + 1] - q0;
-  if (q0 < 0 || q0 + qlen > total_q) {  // a query range outside q: nothing is read or written
+  if (k.b < 0) return k;
+  k.b = __builtin_amdgcn_readfirstlane(k.b);
+  blk = __builtin_amdgcn_readfirstlane(blk);
+  // wave-uniform: scalar registers
+  k.q0 = __builtin_amdgcn_readfirstlane(qo_indptr[k.b]);
+  k.qlen = __builtin_amdgcn_readfirstlane(qo_indptr[k.b + 1]) - k.q0;
+  k.pb = __builtin_amdgcn_readfirstlane(indptr[k.b]);
+  k.npg = max(__builtin_amdgcn_readfirstlane(indptr[k.b + 1]) - k.pb, 0);
+  k.last = __builtin_amdgcn_readfirstlane(min(max(k.npg > 0 ? last_page_len[k.b] : 0, 0), page_size));
+  const int kv_len = k.kv_len = k.npg > 0 ? (k.npg - 1) * page_size + k.last : 0;
+  const int tpp = page_size / kTile;
+  k.r_first = blk * kPfRows;
+  k.r_last = min(k.r_first + kPfRows, k.qlen * group) - 1;
+  k.base_pos = kv_len - k.qlen;  // negative if the cache lacks the new tokens
+  const int kv_end = min(kv_len, max(0, k.base_pos + k.r_last / group + 1));
+  k.ntiles = min((kv_end + kTile - 1) / kTile, k.npg * tpp);
+  // pieces are cut on the sequence's own tokens, so that its row blocks share each piece's K / V
+  const int seq_pairs = (min((kv_len + kTile - 1) / kTile, k.npg * tpp) + 1) / 2;
+  k.piece = max(kPfMinPairs, (seq_pairs + nsplit - 1) / nsplit);
+  k.ns = nsplit > 1 ? max(1, ((k.ntiles + 1) / 2 + k.piece - 1) / k.piece) : 1;
+  return k;
+}
+
+// Grid: row blocks x splits of each KV head. Consecutive workgroups go to the 8 XCDs in turn, so with xcd_per_head > 0
+// the blocks of one KV head run on xcd_per_head XCDs only (their K / V stay in those L2s), and where the splits divide
+// over those XCDs each XCD takes whole splits: every row block that reads a piece of K / V reads it through one L2.
+template <int D>
+__global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefill_kernel(
+    const uint16_t* __restrict__ q, const unsigned char* __restrict__ cache, const int* __restrict__ qo_indptr,
+    const int* __restrict__ indptr, const int* __restrict__ last_page_len, const int* __restrict__ indices,
+    int batch, int total_q, int hq, int hkv, int page_size, int64_t num_pages, float sm_scale, int xcd_per_head,
+    int nblk, int nsplit, int* __restrict__ status, uint16_t* __restrict__ out, const uint16_t* __restrict__ gate,
+    int64_t ldg, float2* __restrict__ part_ml, float* __restrict__ part_o) {
+  using C = PfCfg<D>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int group = hq / hkv;
+  int kvh, want, split;
+  if (xcd_per_head > 0) {
+    const int x = blockIdx.x & 7, sl = blockIdx.x >> 3;
+    kvh = x / xcd_per_head;
+    const int xi = x - kvh * xcd_per_head;
+    if (nsplit % xcd_per_head == 0) {
+      split = sl / nblk * xcd_per_head + xi;
+      want = sl % nblk;
+    } else {
+      const int it = sl * xcd_per_head + xi;
+      split = it / nblk;
+      want = it - split * nblk;
+    }
+  } else {
+    kvh = blockIdx.x % hkv;
+    const int it = blockIdx.x / hkv;
+    split = it / nblk;
+    want = it - split * nblk;
+  }
+  if (split >= nsplit) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, l32 = lane & 31, h = lane >> 5;
+
+  const PfBlock k = pf_block(want, qo_indptr, indptr, last_page_len, batch, group, page_size, nsplit);
+  if (k.b < 0 || split >= k.ns) return;
+  if (k.q0 < 0 || k.q0 + k.qlen > total_q) {  // a query range outside q: nothing is read or written
     if (status && threadIdx.x == 0) *status = 1;
     return;
   }
-  const int pb = indptr[b], npg = max(indptr[b + 1] - pb, 0);
-  const int last = min(max(npg > 0 ? last_page_len[b] : 0, 0), page_size);
-  const int kv_len = npg > 0 ? (npg - 1) * page_size + last : 0;
   const int tpp = page_size / kTile;
-  const int r_first = blk * kPfRows, r_last = min(r_first + kPfRows, qlen * group) - 1;
-  const int base_pos = kv_len - qlen;  // position of new token 0 (negative if the cache lacks the new tokens)
-  const int kv_end = min(kv_len, max(0, base_pos + r_last / group + 1));
-  const int ntiles = min((kv_end + kTile - 1) / kTile, npg * tpp);
-  const float c = sm_scale * kLog2e;
+  // this workgroup's tiles: whole pairs from t_beg, up to t_end
+  const int t_beg = nsplit > 1 ? 2 * split * k.piece : 0;
+  const int t_end = nsplit > 1 ? min(k.ntiles, t_beg + 2 * k.piece) : k.ntiles;
+  // a negative scale moves into Q's signs and a zero scale into zero rows, so that scores keep their order
+  const float sc = sm_scale * kLog2e;
+  const float c = sc == 0.f ? 1.0f : fabsf(sc);
+  const uint32_t flip = sc < 0.f ? 0x80008000u : 0u;
   const int64_t row_stride = (int64_t)hkv * D * 2, plane_stride = (int64_t)page_size * row_stride;
   const uint32_t lds0 = lds_addr(smem);
 
-  // rows of this wave: block i holds row r_first + kPfRowsPerWave wave + 16 i + l16 (replicated over g)
-  int pos[kPfNI];
-  int64_t qoff[kPfNI];
-  axk_bf16x8 qb[kPfNI][C::KSTEPS];
+  // this lane's row (lanes l and l + 32 share it) and its Q as the B operand: elements 16 s + 8 h .. + 7 at step s
+  const int r = k.r_first + 32 * wave + l32;
+  const bool valid = r <= k.r_last;
+  const int rt = valid ? r / group : 0;
+  const int64_t qrow = (int64_t)(k.q0 + rt) * hq + kvh * group + (valid ? r - rt * group : 0);
+  const int pos = valid ? k.base_pos + rt : 0x7fffffff;
+  const uint32_t keep = valid && sc != 0.f ? 0xffffffffu : 0u;
+  axk_u32x4 qw[C::KS];
 #pragma unroll
-  for (int i = 0; i < kPfNI; ++i) {
-    const int r = r_first + kPfRowsPerWave * wave + 16 * i + l16;
-    const bool valid = r <= r_last;
-    const int t = valid ? r / group : 0, h = valid ? r - t * group : 0;
-    pos[i] = valid ? base_pos + t : -1;
-    qoff[i] = ((int64_t)(q0 + t) * hq + kvh * group + h) * D;
-    const uint16_t* qp = q + qoff[i] + 8 * g;
+  for (int s = 0; s < C::KS; ++s) qw[s] = *reinterpret_cast<const axk_u32x4*>(q + qrow * D + 16 * s + 8 * h);
+  axk_bf16x8 qb[C::KS];
 #pragma unroll
-    for (int s = 0; s < C::KSTEPS; ++s) qb[i][s] = valid ? load_bf16x8(qp + 32 * s) : zero_bf16x8();
+  for (int s = 0; s < C::KS; ++s) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qw[s][e] = (qw[s][e] ^ flip) & keep;
+    qb[s] = __builtin_bit_cast(axk_bf16x8, qw[s]);
   }
-  int chunk = 0;
-  int pid = lane < npg ? indices[pb + lane] : 0;
-  asm volatile("" : "+v"(pid));
-#pragma unroll
-  for (int i = 0; i < kPfNI; ++i)
-#pragma unroll
-    for (int s = 0; s < C::KSTEPS; ++s) asm volatile("" : "+v"(qb[i][s]));
+  // the position of the wave's first row (rows are in token order): a pair wholly at or before it needs no mask
+  const int w_first = k.r_first + 32 * wave;
+  const bool active = w_first <= k.r_last;
+  const int pos_lo = k.base_pos + w_first / group;
 
-  auto locate = [&](int ti, int& nvalid) -> const unsigned char* {
-    const int lp = ti / tpp, tp = ti - lp * tpp;
-    if ((lp >> 6) != chunk) {
-      chunk = lp >> 6;
-      const int j = (chunk << 6) + lane;
-      pid = j < npg ? indices[pb + j] : 0;
-      asm volatile("" : "+v"(pid));
-    }
-    int page = __builtin_amdgcn_readlane(pid, lp & 63);  // lp is wave-uniform: a lane read, no LDS round trip
-    const int valid_in_page = (lp == npg - 1) ? last : page_size;
-    nvalid = min(kTile, valid_in_page - tp * kTile);
-    if (page < 0 || page >= num_pages) {
-      if (status && lane == 0 && nvalid > 0) *status = 1;
-      page = 0;
-      nvalid = 0;
-    }
-    return cache + (int64_t)page * 2 * plane_stride + (int64_t)(tp * kTile) * row_stride + (int64_t)kvh * D * 2;
+  // this wave's share of a tile's loads: C::IPW KiB of one plane
+  const int plane = wave * C::IPW / C::IPP, ld_blk = wave * C::IPW % C::IPP;
+  const uint32_t ld_lds = (uint32_t)(plane * C::PLANE + ld_blk * 1024);
+  // lane l holds the address of page 64 chunk + l of the sequence (this KV head, this wave's plane); bad: the lanes
+  // whose page is outside the pool (they hold page 0's)
+  const unsigned char* const head0 = cache + (int64_t)kvh * D * 2 + plane * plane_stride;
+  int chunk = (t_beg / tpp) >> 6;
+  uint32_t pg_lo, pg_hi;
+  unsigned long long bad;
+  auto load_chunk = [&]() {
+    const int j = (chunk << 6) + lane;
+    int pid = j < k.npg ? indices[k.pb + j] : 0;
+    asm volatile("" : "+v"(pid));  // the compiler's wait for this load stays here
+    const bool out_of_pool = pid < 0 || pid >= num_pages;
+    bad = __builtin_amdgcn_ballot_w64(out_of_pool);
+    const uint64_t a = (uint64_t)(uintptr_t)(head0 + (int64_t)(out_of_pool ? 0 : pid) * 2 * plane_stride);
+    pg_lo = (uint32_t)a;
+    pg_hi = (uint32_t)(a >> 32);
   };
+  load_chunk();
+#pragma unroll
+  for (int s = 0; s < C::KS; ++s) asm volatile("" : "+v"(qb[s]));
+
+  // row offsets of this wave's loads inside a tile, and the same clamped to row 0
   int lane_tok[C::IPW];
-  int64_t lane_off[C::IPW], lane_off0[C::IPW];
+  uint32_t lane_off[C::IPW], lane_off0[C::IPW];  // bytes from the tile's first row of that plane
 #pragma unroll
-  for (int k = 0; k < C::IPW; ++k) {
-    const int j = wave * C::IPW + k;
-    const int plane = j / C::IPP, blk2 = j - plane * C::IPP;
-    lane_tok[k] = blk2 * C::RPI + lane / (C::RB / 16);
-    lane_off0[k] = plane * plane_stride + (lane % (C::RB / 16)) * 16;
-    lane_off[k] = lane_off0[k] + (int64_t)lane_tok[k] * row_stride;
+  for (int i = 0; i < C::IPW; ++i) {
+    const int row = (ld_blk + i) * C::RPI + lane / C::NCH, p = lane % C::NCH;
+    lane_tok[i] = row;
+    lane_off0[i] = (uint32_t)((plane ? p ^ (4 * C::vswz(row)) : p ^ C::kswz(row)) * 16);
+    lane_off[i] = lane_off0[i] + (uint32_t)(row * row_stride);
   }
-  auto issue = [&](int ti, int nb) -> int {
-    int nvalid;
-    const unsigned char* kbase = locate(ti < ntiles ? ti : ntiles - 1, nvalid);
-    const int nrow = nvalid > 0 ? nvalid : 1;
-    if (wave < kWaves)  // wave-uniform: the first four waves load the tile
-#pragma unroll
-    for (int k = 0; k < C::IPW; ++k) {
-      const int j = wave * C::IPW + k;
-      const int plane = j / C::IPP, blk2 = j - plane * C::IPP;
-      lds_dma16(kbase + (lane_tok[k] < nrow ? lane_off[k] : lane_off0[k]),
-                lds0 + nb * C::BUF + plane * C::PLANE + blk2 * C::BLK);
+  // the tile cursor: take_pair() gives the tiles two by two, in order (tile cur_tp of page cur_lp): their base
+  // addresses and valid tokens; past t_end the last tile again with no tokens. A page outside the pool holds no tokens
+  // either: its tile is loaded from page 0 and, marked by -kTile tokens, cleared in LDS before use (weight 0 times any
+  // byte of the pool could be NaN). Everything here is wave-uniform. Nearly every pair is two whole tiles of one page
+  // and takes the short path (the general one on every pair: 188 us instead of 179 at 4096 tokens, HQ 16, HKV 2).
+  int cur_ti = t_beg, cur_lp = t_beg / tpp, cur_tp = t_beg - cur_lp * tpp;
+  const int t_whole = min(t_end, k.kv_len / kTile);  // tiles before this one are whole
+  const int64_t tile_stride = kTile * row_stride;
+  auto page_base = [&]() -> const unsigned char* {
+    const uint32_t lo = __builtin_amdgcn_readlane(pg_lo, cur_lp & 63), hi = __builtin_amdgcn_readlane(pg_hi, cur_lp & 63);
+    return reinterpret_cast<const unsigned char*>((uintptr_t)(((uint64_t)hi << 32) | lo)) + cur_tp * tile_stride;
+  };
+  auto take = [&](int& nvalid) -> const unsigned char* {
+    if ((cur_lp >> 6) != chunk) {  // the next 64 pages
+      chunk = cur_lp >> 6;
+      load_chunk();
     }
-    return ti < ntiles ? nvalid : 0;
+    const bool is_bad = (bad >> (cur_lp & 63)) & 1;
+    const int got = min(kTile, (cur_lp == k.npg - 1 ? k.last : page_size) - cur_tp * kTile);
+    if (is_bad && status && lane == 0 && got > 0) *status = 1;
+    nvalid = cur_ti < t_end ? (is_bad ? -kTile : got) : 0;
+    const unsigned char* base = page_base();
+    const int more = cur_ti + 1 < t_end, wrap = more && cur_tp + 1 == tpp;
+    cur_tp = wrap ? 0 : cur_tp + more;
+    cur_lp += wrap;
+    ++cur_ti;
+    return base;
+  };
+  auto take_pair = [&](const unsigned char*& base_a, const unsigned char*& base_b, int& na, int& nb) {
+    if (cur_ti + 2 < t_whole && cur_tp + 2 <= tpp && (cur_lp >> 6) == chunk && !((bad >> (cur_lp & 63)) & 1)) {
+      base_a = page_base();
+      base_b = base_a + tile_stride;
+      na = nb = kTile;
+      cur_ti += 2;  // (a tile follows)
+      const int wrap = cur_tp + 2 == tpp;
+      cur_tp = wrap ? 0 : cur_tp + 2;
+      cur_lp += wrap;
+    } else {
+      base_a = take(na);
+      base_b = take(nb);
+    }
+    base_a = static_cast<const unsigned char*>(uniform_ptr(base_a));
+    base_b = static_cast<const unsigned char*>(uniform_ptr(base_b));
+  };
+  // load i (0 .. IPW - 1) of this wave's share of a tile into the tile slot at `lds`; every address stays inside the
+  // tile's valid rows (a tile past the end has its last tile's rows again: nrow counts those)
+  auto tile_load = [&](auto i, const unsigned char* base, int nrow, uint32_t lds) {
+    constexpr int I = decltype(i)::value;
+    lds_dma16_su_cached<I * 1024>(base, lane_tok[I] < nrow ? lane_off[I] : lane_off0[I], lds + ld_lds);
+  };
+  auto tile_loads = [&](const unsigned char* base, int nrow, uint32_t lds) {
+    tile_load(std::integral_constant<int, 0>{}, base, nrow, lds);
+    if constexpr (C::IPW > 1) tile_load(std::integral_constant<int, 1>{}, base, nrow, lds);
+    if constexpr (C::IPW > 2) tile_load(std::integral_constant<int, 2>{}, base, nrow, lds);
+    if constexpr (C::IPW > 3) tile_load(std::integral_constant<int, 3>{}, base, nrow, lds);
+    static_assert(C::IPW <= 4, "the loads above");
+  };
+  auto clear_tile = [&](int off) {  // this wave's share of a tile slot
+#pragma unroll
+    for (int i = 0; i < C::IPW; ++i)
+      *reinterpret_cast<axk_u32x4*>(smem + off + ld_lds + i * 1024 + lane * 16) = axk_u32x4{0u, 0u, 0u, 0u};
   };
 
-  constexpr int DT = D / 16;
-  axk_f32x4 o[kPfNI][DT];
-  float m_run[kPfNI], l_run[kPfNI];
+  axk_f32x16 o[C::DT];
 #pragma unroll
-  for (int i = 0; i < kPfNI; ++i) {
-    m_run[i] = -INFINITY;
-    l_run[i] = 0.f;
+  for (int t = 0; t < C::DT; ++t)
 #pragma unroll
-    for (int t = 0; t < DT; ++t) o[i][t] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+    for (int i = 0; i < 16; ++i) o[t][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;  // of this lane's row; l_run: this lane's half of the tokens
+  // K row l32 of a pair (row l16 of tile l32 / 16): chunk 2 s + h, its low bits swizzled by the row
+  const int kaddr = (l32 >> 4) * C::BUF + l16 * C::RB + ((h ^ C::kswz(l16)) << 4);
+  // V rows 4 h + l16 / 4 (and + 8) of a tile, bytes 64 t + 32 (lane / 16 % 2) + 8 (l16 % 4)
+  const int vrow = 4 * h + (l16 >> 2);
+  const int vaddr = C::PLANE + vrow * C::RB + 32 * ((lane >> 4) & 1) + 8 * (l16 & 3);
+  const int vx = C::vswz(vrow);
 
-  // the math of tiles ti and ti + 1 (K planes ka, kb; V planes PLANE after them; na, nb valid tokens). The 32 tokens
-  // are one k-step of the 16x16x32 PV MFMA: k = 8 g + j is token 4 g + j of tile ti for j < 4 and token 4 g + j - 4
-  // of tile ti + 1 otherwise, in both operands (P^T from the two score tiles, V^T from one transposing read of each).
+  // One wave a SIMD at D = 256, so the matrix and vector pipes overlap inside the wave: while the probabilities of
+  // pair p are formed from its scores, the scores of pair p + 1 run on MFMA (qk_step); while pair p's P V runs, the
+  // row maxima of pair p + 1 are taken.
+  const axk_f32x16 zero16 = {};
+  auto qk_frag = [&](const unsigned char* buf, int ks) {
+    return *reinterpret_cast<const axk_bf16x8*>(buf + (kaddr ^ (32 * (ks & 7))) + 256 * (ks >> 3));
+  };
+  // the scores of pair p with the tokens past its tiles' valid rows (na, nb) or past the row's position at -inf
+  auto mask = [&](float (&s)[16], int p, int na, int nb) {
+    // token 4 h + 8 (i / 4 % 2) + i % 4 of tile i / 8
+    const int la = min(pos - 32 * p, na - 1) - 4 * h, lb = min(pos - 32 * p - kTile, nb - 1) - 4 * h;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (8 * ((i >> 2) & 1) + (i & 3) > (i < 8 ? la : lb)) s[i] = -INFINITY;
+  };
+  auto row_max = [&](const float (&s)[16]) {
+    float mx = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+    return xor32_max(mx) * c;
+  };
   // The softmax reference max is raised only when a row's scores pass it by more than kPfSlack (log2 units), so
-  // p <= 2^kPfSlack and O is rescaled only on those rare tiles.
+  // p <= 2^kPfSlack and O is rescaled only on those rare pairs.
   constexpr float kPfSlack = 8.0f;
-  // the lowest position among this wave's rows (-1 if it holds an invalid row): a pair of full tiles wholly at or
-  // before it needs no mask (every wave-uniform)
-  int pos_lo = pos[0];
+  auto raise_max = [&](float mx) {
+    const bool raise = mx > m_run + kPfSlack;  // -inf + slack stays -inf: a row's first visible score raises
+    if (__builtin_amdgcn_ballot_w64(raise)) {  // wave-uniform and rare: a branch, not a select per accumulator
+      const float alpha = raise ? __builtin_amdgcn_exp2f(m_run - mx) : 1.0f;
+      if (raise) m_run = mx;
+      l_run *= alpha;
 #pragma unroll
-  for (int i = 1; i < kPfNI; ++i) pos_lo = min(pos_lo, pos[i]);
+      for (int t = 0; t < C::DT; ++t)
 #pragma unroll
-  for (int o2 = 1; o2 < 16; o2 <<= 1) pos_lo = min(pos_lo, __shfl_xor(pos_lo, o2, 64));
-  auto pair_math = [&](const unsigned char* ka, const unsigned char* kb, int ti, int na, int nb, bool full) {
-    axk_f32x4 sa[kPfNI], sb[kPfNI];
-#pragma unroll
-    for (int i = 0; i < kPfNI; ++i) sa[i] = sb[i] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
-    const int roff = C::row_off(l16) + 16 * g;
-#pragma unroll
-    for (int s = 0; s < C::KSTEPS; ++s) {
-      const axk_bf16x8 fa = *reinterpret_cast<const axk_bf16x8*>(ka + roff + 64 * s);
-      const axk_bf16x8 fb = *reinterpret_cast<const axk_bf16x8*>(kb + roff + 64 * s);
-#pragma unroll
-      for (int i = 0; i < kPfNI; ++i) {
-        sa[i] = mfma_bf16_16x16x32(fa, qb[i][s], sa[i]);
-        sb[i] = mfma_bf16_16x16x32(fb, qb[i][s], sb[i]);
-      }
-    }
-    const int tok0 = ti * kTile + 4 * g;
-    axk_bf16x8 pb8[kPfNI];
-    float alpha[kPfNI];
-    bool moved = false;
-#pragma unroll
-    for (int i = 0; i < kPfNI; ++i) {
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        sa[i][rr] *= c;
-        sb[i][rr] *= c;
-      }
-      if (!full) {
-        // token tok0 + rr of tile ti is visible iff rr <= la (inside the tile's valid rows and at or before the
-        // row's position); tile ti + 1 likewise with lb
-        const int la = min(pos[i], ti * kTile + na - 1) - tok0;
-        const int lb = min(pos[i], ti * kTile + kTile + nb - 1) - tok0 - kTile;
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          if (rr > la) sa[i][rr] = -INFINITY;
-          if (rr > lb) sb[i][rr] = -INFINITY;
-        }
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) mx = fmaxf(mx, fmaxf(sa[i][rr], sb[i][rr]));
-      mx = xor32_max(xor16_max(mx));
-      const bool raise = mx > m_run[i] + kPfSlack;  // -inf + slack stays -inf: a row's first visible score raises
-      moved |= __builtin_amdgcn_ballot_w64(raise) != 0;
-      alpha[i] = raise ? __builtin_amdgcn_exp2f(m_run[i] - mx) : 1.0f;
-      if (raise) m_run[i] = mx;
-      // a row that has seen nothing stays at zero: its scores are all -inf and exp2(-inf) = 0
-      const float m_use = m_run[i] == -INFINITY ? 0.f : m_run[i];
-      axk_s16x8 pbits;
-      float psum = 0.f;
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        const float pa = __builtin_amdgcn_exp2f(sa[i][rr] - m_use);
-        const float pbv = __builtin_amdgcn_exp2f(sb[i][rr] - m_use);
-        psum += pa + pbv;
-        pbits[rr] = (short)f32_to_bf16_bits(pa);
-        pbits[4 + rr] = (short)f32_to_bf16_bits(pbv);
-      }
-      pb8[i] = __builtin_bit_cast(axk_bf16x8, pbits);
-      psum = xor32_sum(xor16_sum(psum));
-      l_run[i] = l_run[i] * alpha[i] + psum;
-    }
-    if (moved) {  // wave-uniform and rare: a branch, not a select per accumulator
-#pragma unroll
-      for (int i = 0; i < kPfNI; ++i)
-#pragma unroll
-        for (int t = 0; t < DT; ++t)
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) o[i][t][rr] *= alpha[i];
-    }
-    const int voff = C::PLANE + C::row_off(4 * g + (l16 >> 2)) + 8 * (l16 & 3);
-#pragma unroll
-    for (int t = 0; t < DT; ++t) {
-      const axk_s16x4 va = lds_read_tr16(ka + voff + 32 * t);
-      const axk_s16x4 vb = lds_read_tr16(kb + voff + 32 * t);
-      const axk_bf16x8 v8 = __builtin_bit_cast(axk_bf16x8, __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-      for (int i = 0; i < kPfNI; ++i) o[i][t] = mfma_bf16_16x16x32(v8, pb8[i], o[i][t]);
+        for (int i = 0; i < 16; ++i) o[t][i] *= alpha;
     }
   };
 
-  if (ntiles > 0) {
-    // tiles land kPfAhead ahead in a ring of kPfBuf = kPfAhead + 2; an iteration computes two
-    int nv[kPfAhead];  // valid tokens of tiles ti .. ti + kPfAhead - 1
+  if (t_end > t_beg) {
+    // One MFMA a stage, with the LDS reads of a later stage's fragment, a share of the vector work and one of the next
+    // pair's loads beside it: K fragments are read KA stages ahead, V fragments VA. The compiler orders inside a stage
+    // only (left to itself it waits for nearly every fragment right after reading it: 187 us against 178 at 4096
+    // tokens; the loads before the stages instead of among them: 200 us).
+    constexpr int KA = C::KS / 4, PV = 2 * C::DT, VA = C::DT / 2, EX0 = 4, EXS = C::KS * 3 / 4;
+    static_assert(2 * C::IPW <= C::KS, "a pair's loads fit the score stages");
+    constexpr int AHEAD = kPfRing - 1;  // pairs in flight
+    int na[AHEAD], nb[AHEAD];           // the valid tokens of their tiles
+    auto rows_of = [&](int n) { return n > 0 ? n : 1; };
 #pragma unroll
-    for (int j = 0; j < kPfAhead; ++j) nv[j] = issue(j, j);
-    for (int ti = 0; ti < ntiles; ti += 2) {
-      wait_vmcnt<(kPfAhead - 2) * C::IPW>();  // this wave's loads of tiles ti, ti + 1 have landed
-      __builtin_amdgcn_s_barrier();            // ... and every wave's; all are done with tiles ti - 2, ti - 1
-      const int n0 = issue(ti + kPfAhead, (ti + kPfAhead) % kPfBuf);  // into the buffers of tiles ti - 2, ti - 1
-      const int n1 = issue(ti + kPfAhead + 1, (ti + kPfAhead + 1) % kPfBuf);
-      const int na = nv[0], nb = nv[1];
+    for (int j = 0; j < AHEAD; ++j) {
+      const unsigned char *ba, *bb;
+      take_pair(ba, bb, na[j], nb[j]);
+      tile_loads(ba, rows_of(na[j]), lds0 + j * C::PAIR);
+      tile_loads(bb, rows_of(nb[j]), lds0 + j * C::PAIR + C::BUF);
+    }
+    const int p_beg = t_beg / 2, p_end = (t_end + 1) / 2;
+    // the pair with tokens (a, b) in ring slot sl has landed for every wave: clear its tiles of pages outside the pool
+    auto clear_bad = [&](int a, int b, int sl) {
+      if (a >= 0 && b >= 0) return;
+      if (a < 0) clear_tile(sl * C::PAIR);
+      if (b < 0) clear_tile(sl * C::PAIR + C::BUF);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+    };
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kPfRing - 2) * 2 * C::IPW) : "memory");
+    __builtin_amdgcn_s_barrier();  // every wave's loads of the first pair have landed
+    clear_bad(na[0], nb[0], 0);
+    int slot = 0, slot_n;  // of pairs p and p + 1
+    uint32_t dst;          // the slot of pair p - 1, which takes pair p + AHEAD
+    const unsigned char *base_a, *base_b;
+    int ra, rb;
+    auto advance = [&]() {  // to pair p: every wave's loads of pair p + 1 have landed, and its reads of pair p - 1 are done
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kPfRing - 3) * 2 * C::IPW) : "memory");
+      __builtin_amdgcn_s_barrier();
+      slot_n = slot + 1 == kPfRing ? 0 : slot + 1;
+      dst = lds0 + (slot == 0 ? kPfRing - 1 : slot - 1) * C::PAIR;
 #pragma unroll
-      for (int j = 0; j + 2 < kPfAhead; ++j) nv[j] = nv[j + 2];
-      nv[kPfAhead - 2] = n0;
-      nv[kPfAhead - 1] = n1;
-      unsigned char* ka = smem + (ti % kPfBuf) * C::BUF;
-      unsigned char* kb = smem + ((ti + 1) % kPfBuf) * C::BUF;
-      const bool full = na == kTile && nb == kTile && ti * kTile + 2 * kTile - 1 <= pos_lo;
-      if (na + nb > 0) pair_math(ka, kb, ti, na, nb, full);
+      for (int j = 0; j + 1 < AHEAD; ++j) na[j] = na[j + 1], nb[j] = nb[j + 1];
+      clear_bad(na[0], nb[0], slot_n);
+      take_pair(base_a, base_b, na[AHEAD - 1], nb[AHEAD - 1]);
+      ra = rows_of(na[AHEAD - 1]), rb = rows_of(nb[AHEAD - 1]);
+    };
+    if (!active) {  // no rows (the end of a row block): this wave only loads its share
+      for (int p = p_beg; p < p_end; ++p) {
+        advance();
+        tile_loads(base_a, ra, dst);
+        tile_loads(base_b, rb, dst + C::BUF);
+        slot = slot_n;
+      }
+      wait_vmcnt<0>();
+      return;
+    }
+    float s[16];
+    {
+      axk_f32x16 sn = zero16;
+#pragma unroll
+      for (int ks = 0; ks < C::KS; ++ks) sn = mfma_bf16_32x32x16(qk_frag(smem, ks), qb[ks], sn);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = sn[i];
+      if (na[0] != kTile || nb[0] != kTile || 32 * p_beg + 31 > pos_lo) mask(s, p_beg, na[0], nb[0]);
+      raise_max(row_max(s));
+    }
+    for (int p = p_beg; p < p_end; ++p) {
+      advance();
+      {
+        const unsigned char* kb = smem + slot_n * C::PAIR;
+        const unsigned char* vb = smem + slot * C::PAIR;
+        auto pv_frag = [&](int j) {  // V^T tile j mod DT of the pair's 16-token tile j / DT
+          const int t = j % C::DT;
+          const unsigned char* va = vb + vaddr + 64 * ((t & 3) ^ vx) + 256 * (t >> 2) + (j / C::DT) * C::BUF;
+          const axk_s16x4 v0 = lds_read_tr16(va), v1 = lds_read_tr16(va + 8 * C::RB);
+          return __builtin_bit_cast(axk_bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        // a row that has seen nothing stays at zero: its scores are all -inf and exp2(-inf) = 0
+        const float m_use = m_run == -INFINITY ? 0.f : m_run;
+        axk_f32x16 sn = zero16;
+        axk_bf16x8 kf[KA], vf[VA], pf[2];
+        auto probs = [&](int lo, int hi) {
+#pragma unroll
+          for (int i = lo; i < hi; ++i) {
+            s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -m_use));
+            l_run += s[i];
+          }
+          asm volatile("" : "+v"(l_run));  // the sum stays in this stage
+        };
+#pragma unroll
+        for (int i = 0; i < KA; ++i) kf[i] = qk_frag(kb, i);
+        probs(0, EX0);
+        __builtin_amdgcn_sched_barrier(0);
+        auto qk_stage = [&](auto stage) {
+          constexpr int I = decltype(stage)::value;
+          sn = mfma_bf16_32x32x16(kf[I % KA], qb[I], sn);
+          asm volatile("" : "+a"(sn));  // this MFMA stays in this stage (and the accumulators in AGPRs)
+          if constexpr (I + KA < C::KS) kf[I % KA] = qk_frag(kb, I + KA);
+          else if constexpr (I + KA - C::KS < VA) vf[I + KA - C::KS] = pv_frag(I + KA - C::KS);
+          if constexpr (I < C::IPW) tile_load(std::integral_constant<int, I % C::IPW>{}, base_a, ra, dst);
+          else if constexpr (I < 2 * C::IPW)
+            tile_load(std::integral_constant<int, I % C::IPW>{}, base_b, rb, dst + C::BUF);
+          if constexpr (I < EXS) probs(EX0 + I * (16 - EX0) / EXS, EX0 + (I + 1) * (16 - EX0) / EXS);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        for_each_index<C::KS>(qk_stage);
+#pragma unroll
+        for (int i = KA; i < VA; ++i) vf[i] = pv_frag(i);
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti) {
+          axk_u32x4 w;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(s[8 * ti + 2 * i], s[8 * ti + 2 * i + 1]);
+          pf[ti] = __builtin_bit_cast(axk_bf16x8, w);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < PV; ++j) {
+          o[j % C::DT] = mfma_bf16_32x32x16(vf[j % VA], pf[j / C::DT], o[j % C::DT]);
+          asm volatile("" : "+a"(o[j % C::DT]));
+          if (j + VA < PV) vf[j % VA] = pv_frag(j + VA);
+          if (j >= 2)
+#pragma unroll
+            for (int i = 16 * (j - 2) / (PV - 2); i < 16 * (j - 1) / (PV - 2); ++i) {
+              s[i] = sn[i];
+              asm volatile("" : "+v"(s[i]));  // one copy out of the accumulator
+              mx = fmaxf(mx, s[i]);
+            }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        mx = xor32_max(mx) * c;
+        if (na[0] != kTile || nb[0] != kTile || 32 * p + 63 > pos_lo) {
+          mask(s, p + 1, na[0], nb[0]);
+          mx = row_max(s);
+        }
+        raise_max(mx);
+      }
+      slot = slot_n;
     }
     wait_vmcnt<0>();
   }
 
-  // lane (row l16 of block i, g) holds O[row][d = 16 t + 4 g .. + 3]
+  // lane (row, half h) holds O[row][d = 32 t + 8 (i / 4) + 4 h + i % 4]
+  l_run = xor32_sum(l_run);
+  if (!valid) return;
+  if (k.ns > 1) {
+    const int64_t slot = (int64_t)split * total_q * hq + qrow;
+    if (h == 0) part_ml[slot] = make_float2(m_run, l_run);
 #pragma unroll
-  for (int i = 0; i < kPfNI; ++i) {
-    const int r = r_first + kPfRowsPerWave * wave + 16 * i + l16;
-    if (r > r_last) continue;
-    const float inv = l_run[i] > 0.f ? 1.0f / l_run[i] : 0.f;
-    const int64_t gi0 = qoff[i] / D * ldg;  // the row's gate (with a gate)
+    for (int t = 0; t < C::DT; ++t)
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
-      const int col = 16 * t + 4 * g;
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(part_o + slot * D + 32 * t + 8 * i + 4 * h) =
+            make_float4(o[t][4 * i], o[t][4 * i + 1], o[t][4 * i + 2], o[t][4 * i + 3]);
+    return;
+  }
+  const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+#pragma unroll
+  for (int t = 0; t < C::DT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int col = 32 * t + 8 * i + 4 * h;
+      const int64_t gi = qrow * ldg + col;  // (with a gate)
       uint2 w;
-      w.x = gated_bf16(o[i][t][0] * inv, gate, gi0 + col) | (gated_bf16(o[i][t][1] * inv, gate, gi0 + col + 1) << 16);
-      w.y = gated_bf16(o[i][t][2] * inv, gate, gi0 + col + 2) | (gated_bf16(o[i][t][3] * inv, gate, gi0 + col + 3) << 16);
-      *reinterpret_cast<uint2*>(out + qoff[i] + col) = w;
+      w.x = gated_bf16(o[t][4 * i] * inv, gate, gi) | (gated_bf16(o[t][4 * i + 1] * inv, gate, gi + 1) << 16);
+      w.y = gated_bf16(o[t][4 * i + 2] * inv, gate, gi + 2) | (gated_bf16(o[t][4 * i + 3] * inv, gate, gi + 3) << 16);
+      *reinterpret_cast<uint2*>(out + qrow * D + col) = w;
+    }
+}
+
+// The log-sum-exp merge of the splits of each row (as paged_merge_kernel): one wave per row, kPfMergeRows rows of one
+// row block per workgroup. Row blocks with a single split wrote their output already.
+template <int D>
+__global__ __launch_bounds__(256) void paged_prefill_merge_kernel(
+    const int* __restrict__ qo_indptr, const int* __restrict__ indptr, const int* __restrict__ last_page_len,
+    int batch, int total_q, int hq, int hkv, int page_size, int nsplit, const float2* __restrict__ part_ml,
+    const float* __restrict__ part_o, uint16_t* __restrict__ out, const uint16_t* __restrict__ gate, int64_t ldg) {
+  constexpr int PER = D / 64;  // columns per lane
+  const int group = hq / hkv;
+  constexpr int SUB = kPfRows / kPfMergeRows;
+  const int sub = blockIdx.x % SUB, kvh = blockIdx.x / SUB % hkv, want = blockIdx.x / SUB / hkv;
+  const PfBlock k = pf_block(want, qo_indptr, indptr, last_page_len, batch, group, page_size, nsplit);
+  if (k.b < 0 || k.ns <= 1 || k.q0 < 0 || k.q0 + k.qlen > total_q) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int i = wave; i < kPfMergeRows; i += 4) {
+    const int r = k.r_first + sub * kPfMergeRows + i;
+    if (r > k.r_last) return;
+    const int rt = r / group;
+    const int64_t qrow = (int64_t)(k.q0 + rt) * hq + kvh * group + (r - rt * group);
+    const int64_t step = (int64_t)total_q * hq;
+    const float2 ml = lane < k.ns ? part_ml[lane * step + qrow] : make_float2(-INFINITY, 0.f);
+    const float m = wave_max(ml.x);
+    const float w = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - m);
+    const float l = wave_sum(ml.y * w);
+    float acc[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) acc[e] = 0.f;
+    const float* po = part_o + qrow * D + lane * PER;
+    for (int j0 = 0; j0 < k.ns; j0 += 8) {  // eight splits' loads in flight
+      float v[8][PER];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < PER; ++e) v[j][e] = po[min(j0 + j, k.ns - 1) * step * D + e];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float wj = j0 + j < k.ns ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+                                             __builtin_bit_cast(int, w), min(j0 + j, 63))) : 0.f;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) acc[e] = fmaf(v[j][e], wj, acc[e]);
+      }
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int col = lane * PER + e;
+      out[qrow * D + col] = (uint16_t)gated_bf16(acc[e] * inv, gate, qrow * ldg + col);
     }
   }
+}
+
+// KV splits of a prefill call: enough that the row blocks of all sequences and KV heads fill the chip's 256 workgroup
+// slots (one a CU at D = 256), none where they fill half of them already: a split row block writes and reads back
+// its fp32 partials (1 KiB a row and split at D = 256). A sequence shorter than kPfMinPairs pairs a split gets fewer
+// (pf_block), down to the unsplit form.
+int pf_splits(int64_t batch, int64_t total_q, int64_t hq, int64_t hkv) {
+  const int64_t blocks = std::max(batch, (total_q * (hq / hkv) + kPfRows - 1) / kPfRows) * hkv;
+  int ns = 1;
+  while (ns < kPfMaxSplits && blocks * ns * 2 <= kPfSlots) ns *= 2;
+  return ns;
+}
+
+size_t pf_ws_bytes(int64_t batch, int64_t total_q, int64_t hq, int64_t hkv, int64_t d) {
+  const int ns = pf_splits(batch, total_q, hq, hkv);
+  return ns > 1 ? (size_t)ns * total_q * hq * (sizeof(float2) + sizeof(float) * d) : 0;
 }
 
 template <int D>
 int launch_prefill(const uint16_t* q, const void* cache, const int* qo_indptr, const int* indptr, const int* last,
                    const int* indices, uint16_t* out, int batch, int total_q, int hq, int hkv, int page_size,
-                   int64_t num_pages, float sm_scale, int* status, hipStream_t st, const uint16_t* gate = nullptr,
-                   int64_t ldg = 0) {
+                   int64_t num_pages, float sm_scale, int* status, hipStream_t st, const uint16_t* gate, int64_t ldg,
+                   void* ws) {
   const int64_t rows = (int64_t)total_q * (hq / hkv);
-  const int64_t nblk = (rows + kPfRows - 1) / kPfRows + batch;  // >= the sum over sequences of their row blocks
-  const int xph = hkv <= 8 && 8 % hkv == 0 ? 8 / hkv : 0;      // XCDs per KV head
-  const int64_t grid = xph ? 8 * ((nblk + xph - 1) / xph) : nblk * hkv;
+  const int ns = ws ? pf_splits(batch, total_q, hq, hkv) : 1;
+  // >= the sum over sequences of their row blocks (one sequence: exactly)
+  const int64_t nblk = (rows + kPfRows - 1) / kPfRows + (batch > 1 ? batch : 0);
+  const int xph = hkv <= 8 && 8 % hkv == 0 ? 8 / hkv : 0;  // XCDs per KV head
+  const int64_t grid = xph ? 8 * ((nblk * ns + xph - 1) / xph) : nblk * ns * hkv;
   if (grid > 0x7fffffff) return AXK_E_SHAPE;
-  const size_t lds = (size_t)kPfBuf * PagedCfg<D>::BUF;
+  const size_t lds = (size_t)kPfRing * PfCfg<D>::PAIR;
   static AxkOnce lds_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
   if (const int rc = axk_raise_lds(lds_once, reinterpret_cast<const void*>(&paged_prefill_kernel<D>), lds)) return rc;
+  float2* ml = static_cast<float2*>(ws);
+  float* po = reinterpret_cast<float*>(ml + (ws ? (int64_t)ns * total_q * hq : 0));
   AXK_LAUNCH_GATE();
   hipLaunchKernelGGL((paged_prefill_kernel<D>), dim3((unsigned)grid), dim3(64 * kPfWaves), lds, st, q,
                      static_cast<const unsigned char*>(cache), qo_indptr, indptr, last, indices, batch, total_q, hq,
-                     hkv, page_size, num_pages, sm_scale, xph, status, out, gate, ldg);
+                     hkv, page_size, num_pages, sm_scale, xph, (int)nblk, ns, status, out, gate, ldg, ml, po);
+  if (ns > 1)
+    hipLaunchKernelGGL((paged_prefill_merge_kernel<D>), dim3((unsigned)(nblk * hkv * (kPfRows / kPfMergeRows))),
+                       dim3(256), 0, st, qo_indptr, indptr, last, batch, total_q, hq, hkv, page_size, ns, ml, po, out,
+                       gate, ldg);
   return axk_launch_status();
 }
 
@@ -1989,7 +2287,8 @@ namespace {
 int prefill_impl(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr, const int32_t* indptr,
                  const int32_t* indices, const int32_t* last_page_len, uint16_t* out, int64_t batch, int64_t total_q,
                  int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages,
-                 float sm_scale, int32_t* status, hipStream_t st, const uint16_t* gate, int64_t ldg) {
+                 float sm_scale, int32_t* status, hipStream_t st, const uint16_t* gate, int64_t ldg, void* workspace,
+                 size_t workspace_bytes) {
   AXK_REQUIRE(q && kv_cache && qo_indptr && indptr && indices && last_page_len && out, AXK_E_NULL);
   AXK_REQUIRE(batch > 0 && batch <= (1 << 20) && total_q >= 0 && total_q <= (1 << 24), AXK_E_SHAPE);
   AXK_REQUIRE(num_kv_heads > 0 && num_qo_heads > 0 && num_qo_heads % num_kv_heads == 0, AXK_E_SHAPE);
@@ -2000,17 +2299,21 @@ int prefill_impl(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_
   if (total_q == 0) return AXK_OK;
   const size_t qbytes = (size_t)total_q * num_qo_heads * head_dim * 2;
   AXK_REQUIRE(!axk_overlap(out, qbytes, q, qbytes), AXK_E_ALIAS);
+  const size_t need = pf_ws_bytes(batch, total_q, num_qo_heads, num_kv_heads, head_dim);
+  AXK_REQUIRE(!workspace || axk_aligned(workspace, 16), AXK_E_ALIGN);
+  void* ws = need > 0 && workspace_bytes >= need ? workspace : nullptr;
+  AXK_REQUIRE(!ws || (!axk_overlap(ws, need, out, qbytes) && !axk_overlap(ws, need, q, qbytes)), AXK_E_ALIAS);
   const int B = (int)batch, T = (int)total_q, HQ = (int)num_qo_heads, HKV = (int)num_kv_heads, PS = (int)page_size;
   switch (head_dim) {
     case 64:
       return launch_prefill<64>(q, kv_cache, qo_indptr, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
-                                num_pages, sm_scale, status, st, gate, ldg);
+                                num_pages, sm_scale, status, st, gate, ldg, ws);
     case 128:
       return launch_prefill<128>(q, kv_cache, qo_indptr, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
-                                 num_pages, sm_scale, status, st, gate, ldg);
+                                 num_pages, sm_scale, status, st, gate, ldg, ws);
     default:
       return launch_prefill<256>(q, kv_cache, qo_indptr, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
-                                 num_pages, sm_scale, status, st, gate, ldg);
+                                 num_pages, sm_scale, status, st, gate, ldg, ws);
   }
 }
 }  // namespace
@@ -2021,14 +2324,39 @@ extern "C" int axk_paged_prefill(const uint16_t* q, const uint16_t* kv_cache, co
                                  int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages,
                                  float sm_scale, int32_t* status, axk_stream_t stream) {
   return prefill_impl(q, kv_cache, qo_indptr, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
-                      num_kv_heads, head_dim, page_size, num_pages, sm_scale, status, axk_stream(stream), nullptr, 0);
+                      num_kv_heads, head_dim, page_size, num_pages, sm_scale, status, axk_stream(stream), nullptr, 0,
+                      nullptr, 0);
+}
+
+extern "C" size_t axk_paged_prefill_workspace_size(int64_t batch, int64_t total_q, int64_t num_qo_heads,
+                                                   int64_t num_kv_heads, int64_t head_dim) {
+  if (batch <= 0 || batch > (1 << 20) || total_q <= 0 || total_q > (1 << 24) || num_kv_heads <= 0 ||
+      num_qo_heads <= 0 || num_qo_heads % num_kv_heads != 0 || num_kv_heads > 4096 ||
+      total_q * num_qo_heads > ((int64_t)1 << 31) / 256 || !(head_dim == 64 || head_dim == 128 || head_dim == 256))
+    return 0;
+  return pf_ws_bytes(batch, total_q, num_qo_heads, num_kv_heads, head_dim);
+}
+
+extern "C" int axk_paged_prefill_split(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr,
+                                       const int32_t* indptr, const int32_t* indices, const int32_t* last_page_len,
+                                       uint16_t* out, int64_t batch, int64_t total_q, int64_t num_qo_heads,
+                                       int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages,
+                                       float sm_scale, int32_t* status, void* workspace, size_t workspace_bytes,
+                                       axk_stream_t stream) {
+  AXK_REQUIRE(workspace_bytes >=
+                  axk_paged_prefill_workspace_size(batch, total_q, num_qo_heads, num_kv_heads, head_dim),
+              AXK_E_WORKSPACE);
+  return prefill_impl(q, kv_cache, qo_indptr, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
+                      num_kv_heads, head_dim, page_size, num_pages, sm_scale, status, axk_stream(stream), nullptr, 0,
+                      workspace, workspace_bytes);
 }
 
 int axk_paged_prefill_gated(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr,
                             const int32_t* indptr, const int32_t* indices, const int32_t* last_page_len,
                             const uint16_t* gate, int64_t ldg, uint16_t* out, int64_t batch, int64_t total_q,
                             int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
-                            int64_t num_pages, float sm_scale, hipStream_t stream) {
+                            int64_t num_pages, float sm_scale, void* workspace, size_t workspace_bytes,
+                            hipStream_t stream) {
   AXK_REQUIRE(gate, AXK_E_NULL);
   AXK_REQUIRE(ldg >= head_dim, AXK_E_SHAPE);
   if (total_q > 0) {
@@ -2036,5 +2364,6 @@ int axk_paged_prefill_gated(const uint16_t* q, const uint16_t* kv_cache, const i
     AXK_REQUIRE(!axk_overlap(out, (size_t)total_q * num_qo_heads * head_dim * 2, gate, gbytes), AXK_E_ALIAS);
   }
   return prefill_impl(q, kv_cache, qo_indptr, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
-                      num_kv_heads, head_dim, page_size, num_pages, sm_scale, nullptr, stream, gate, ldg);
+                      num_kv_heads, head_dim, page_size, num_pages, sm_scale, nullptr, stream, gate, ldg, workspace,
+                      workspace_bytes);
 }

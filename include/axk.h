@@ -360,6 +360,19 @@ int axk_paged_prefill(const uint16_t* q, const uint16_t* kv_cache, const int32_t
                       int64_t total_q, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
                       int64_t page_size, int64_t num_pages, float sm_scale, int32_t* status, axk_stream_t stream);
 
+/* axk_paged_prefill with each sequence's cached tokens split over several workgroups, for calls whose row blocks (128
+ * rows of total_q x num_qo_heads / num_kv_heads, per KV head) would leave the chip idle: a prefill page or draft rows
+ * over a long history. The splits' fp32 partials live in workspace (16-byte aligned, axk_paged_prefill_workspace_size
+ * bytes, overlapping nothing else; 0 when the call would not split: workspace may then be NULL). Otherwise as
+ * axk_paged_prefill. */
+size_t axk_paged_prefill_workspace_size(int64_t batch, int64_t total_q, int64_t num_qo_heads, int64_t num_kv_heads,
+                                        int64_t head_dim);
+int axk_paged_prefill_split(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr,
+                            const int32_t* indptr, const int32_t* indices, const int32_t* last_page_len, uint16_t* out,
+                            int64_t batch, int64_t total_q, int64_t num_qo_heads, int64_t num_kv_heads,
+                            int64_t head_dim, int64_t page_size, int64_t num_pages, float sm_scale, int32_t* status,
+                            void* workspace, size_t workspace_bytes, axk_stream_t stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Gated DeltaNet (GDN)
  * ------------------------------------------------------------------------------------------- */
