@@ -391,8 +391,9 @@ int group_dispatch(const uint16_t* a, int64_t lda, const MxGroup& g, int64_t m, 
 }
 
 // ---------------------------------------------------------------------------------------------
-// The large-M path (prefill): a dense GEMM over the matrices of a group (or a gate / up pair) with an LDS pipeline.
-// Workgroup = BM activation rows (dg_bm: 128 for MXFP4, 64 for the 8-bit formats) x 256 weight rows (EPI_SWIGLU: 128
+// The large-M path (prefill, and fewer rows of wide matrices: dg_rows): a dense GEMM over the matrices of a group (or a
+// gate / up pair) with an LDS pipeline. Workgroup = BM activation rows (dg_bm: 128 for the 4-bit formats, 64 for the
+// 8-bit ones; less where that leaves CUs without a workgroup: dg_epi) x 256 weight rows (EPI_SWIGLU: 128
 // gate + the same 128 up channels), wave w a BM x 64 block of BM / 16 by four MFMA tiles (every A fragment feeds
 // four MFMAs, every decoded B fragment BM / 16). The activation rows and the
 // weight rows of each 64-wide K step land in a ring of kDgStages LDS slots by direct loads two steps ahead, one
@@ -404,28 +405,22 @@ int group_dispatch(const uint16_t* a, int64_t lda, const MxGroup& g, int64_t m, 
 // kernel's. Consecutive workgroups go round-robin over the 8 XCDs, so each XCD takes a contiguous run of the tile
 // order, which walks groups of 8 row blocks across all column blocks: an XCD's L2 keeps its activation rows.
 // ---------------------------------------------------------------------------------------------
-constexpr int kDgBN = 256, kDgBK = 64, kDgStages = 3, kDgXcds = 8, kDgGroupRows = 8;
+constexpr int kDgBN = 256, kDgBK = 64, kDgStages = 3, kDgXcds = 8, kDgGroupRows = 8, kDgCus = 256;
 // activation rows per workgroup: 128 for MXFP4 (each decoded weight fragment feeds eight MFMAs; a 75 KiB ring, two
 // workgroups a CU), 64 for the 8-bit formats (whose 64-byte weight rows would make a 128-row ring 99 KiB: one a CU)
 template <int F>
 constexpr int dg_bm() { return axk::is_fp4(F) ? 128 : 64; }
-template <int F>
-constexpr int dg_mt() { return dg_bm<F>() / 16; }  // 16-row MFMA tiles per wave (a wave spans every row of the tile)
-template <int F>
-constexpr int dg_ai() { return dg_bm<F>() * kDgBK * 2 / 1024 / 4; }  // A direct-load instructions per wave and step
-template <int F>
-constexpr int dg_astage() { return dg_bm<F>() * kDgBK * 2; }
-constexpr int64_t kDgMinRows = 128;  // below this the group kernel (weights streamed once per 16 / 32 rows) is faster
+constexpr int64_t kDgMinRows = 128;  // from here on the dense GEMM takes every width
 template <int F>
 constexpr int dg_row_bytes() { return axk::is_fp4(F) ? kDgBK / 2 : kDgBK; }  // weight bytes per row and step
 constexpr int kDgSStage = kDgBN * 4;  // MX formats: one scale dword per weight row and step
-template <int F>
+template <int F, int BM>
 constexpr int dg_stage() {
-  return dg_astage<F>() + kDgBN * dg_row_bytes<F>() + (axk::has_block_scales(F) ? kDgSStage : 0);
+  return BM * kDgBK * 2 + kDgBN * dg_row_bytes<F>() + (axk::has_block_scales(F) ? kDgSStage : 0);
 }
-template <int F>
-size_t dg_lds_bytes(int64_t) {
-  return (size_t)kDgStages * dg_stage<F>();
+template <int F, int BM>
+constexpr int dg_lds_bytes() {
+  return kDgStages * dg_stage<F, BM>();
 }
 
 struct DgArgs {
@@ -448,26 +443,32 @@ struct DgArgs {
   int m, k;
 };
 
+// A lane's 16 weights of a 64-wide step, k = 16 g4 .. + 15 of the row (one LDS read, one block scale), as the B operands
+// of the step's two MFMAs: MFMA kh takes k = 16 g4 + 8 kh + j for its index (g4, j), in both operands.
 template <int F>
-AXK_DEV axk_bf16x8 dg_decode(const unsigned char* row, int kh, int g4, int r, float sc) {
+AXK_DEV void dg_decode(const unsigned char* row, int g4, int r, float sc, axk_bf16x8 (&out)[2]) {
   if constexpr (axk::is_fp4(F)) {
-    const uint32_t w = *reinterpret_cast<const uint32_t*>(row + 16 * (kh ^ ((r >> 3) & 1)) + 4 * g4);
-    if constexpr (F == axk::WF_NVFP4) return fp4x8_to_bf16x8_mul(w, sc);
-    else return fp4x8_to_bf16x8(w, sc);
+    const uint2 w = *reinterpret_cast<const uint2*>(row + 16 * ((g4 >> 1) ^ ((r >> 3) & 1)) + 8 * (g4 & 1));
+    if constexpr (F == axk::WF_NVFP4) {
+      out[0] = fp4x8_to_bf16x8_mul(w.x, sc);
+      out[1] = fp4x8_to_bf16x8_mul(w.y, sc);
+    } else {
+      out[0] = fp4x8_to_bf16x8(w.x, sc);
+      out[1] = fp4x8_to_bf16x8(w.y, sc);
+    }
   } else {
-    // 8 bytes (k = 32 kh + 8 g4 ..) of the 64-byte row: chunk 2 kh + g4 / 2, half g4 % 2
-    const int c = (2 * kh + (g4 >> 1)) ^ ((r >> 2) & 3);
-    const uint2 w = *reinterpret_cast<const uint2*>(row + 16 * c + 8 * (g4 & 1));
-    const uint4 q = make_uint4(w.x, w.y, 0u, 0u);
-    return axk::WUnit<F>::conv(q, 0, sc);
+    const uint4 w = *reinterpret_cast<const uint4*>(row + 16 * (g4 ^ ((r >> 2) & 3)));
+    out[0] = axk::WUnit<F>::conv(w, 0, sc);
+    out[1] = axk::WUnit<F>::conv(w, 1, sc);
   }
 }
 
-template <int F, int EPI>
+template <int F, int EPI, int BM>
 __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int RB = dg_row_bytes<F>(), STAGE = dg_stage<F>();
-  constexpr int kDgBM = dg_bm<F>(), kDgMT = dg_mt<F>(), kDgAI = dg_ai<F>(), kDgAStage = dg_astage<F>();
+  constexpr int RB = dg_row_bytes<F>(), STAGE = dg_stage<F, BM>();
+  constexpr int ST = kDgStages, kDgBM = BM, kDgMT = BM / 16;  // 16-row MFMA tiles per wave (a wave spans every row of the tile)
+  constexpr int kDgAStage = BM * kDgBK * 2, kDgAI = kDgAStage / 1024 / 4;  // A direct loads per wave and step
   constexpr int COLS = EPI == EPI_SWIGLU ? kDgBN / 2 : kDgBN;  // output channels per workgroup
   const int nb = EPI == EPI_PLAIN ? g.cb0[g.count] : (g.n[0] + COLS - 1) / COLS, mb = (g.m + kDgBM - 1) / kDgBM;
   const int total = nb * mb, per = (total + kDgXcds - 1) / kDgXcds;
@@ -530,10 +531,9 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
   const uint8_t* ssrc = axk::has_block_scales(F) ? wrow(64 * wave + lane, true) : nullptr;
   // step ks into ring slot BUF (past the last step the last one again: in bounds, unused), so every iteration
   // waits on the same count
-  auto issue = [&](int ks, auto buf_c) __attribute__((always_inline)) {
-    constexpr int BUF = decltype(buf_c)::value;
+  auto issue = [&](int ks, int buf) __attribute__((always_inline)) {
     const int kk = min(ks, nk - 1);
-    const uint32_t base = lds0 + BUF * STAGE;
+    const uint32_t base = lds0 + buf * STAGE;
 #pragma unroll
     for (int h = 0; h < kDgAI; ++h) lds_dma16_cached(asrc[h] + kk * kDgBK, base + (kDgAI * wave + h) * 1024);
 #pragma unroll
@@ -543,50 +543,81 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
     if constexpr (axk::is_nv(F)) lds_dma4_cached(ssrc + 4 * kk, base + kDgAStage + kDgBN * RB + 256 * wave);
   };
   constexpr int LPS = kDgAI + BI + (axk::has_block_scales(F) ? 1 : 0);  // vector-memory instructions per step
-  issue(0, std::integral_constant<int, 0>{});
-  issue(1, std::integral_constant<int, 1>{});
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i) issue(i, i);
   axk_f32x4 acc[kDgMT][4];
 #pragma unroll
   for (int mt = 0; mt < kDgMT; ++mt)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[mt][j] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto step = [&](int ks, auto buf_c) __attribute__((always_inline)) {
-    constexpr int BUF = decltype(buf_c)::value;
-    wait_vmcnt<LPS>();  // this wave's loads of step ks have landed (step ks + 1's may not have)
+  auto step = [&](int ks, int buf) __attribute__((always_inline)) {
+    wait_vmcnt<(ST - 2) * LPS>();  // this wave's loads of step ks have landed (those of later steps may not have)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of step ks - 1 are done
     __builtin_amdgcn_s_barrier();  // every wave's step-ks loads landed; every wave is done with step ks - 1
     asm volatile("" ::: "memory");
-    issue(ks + 2, std::integral_constant<int, (BUF + 2) % kDgStages>{});  // into the slot of step ks - 1
-    const unsigned char* sa = smem + BUF * STAGE;
+    issue(ks + ST - 1, buf == 0 ? ST - 1 : buf - 1);  // into the slot of step ks - 1
+    const unsigned char* sa = smem + buf * STAGE;
     const unsigned char* sb = sa + kDgAStage;
+    axk_bf16x8 bf[4][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = brow[j] + l16;
+      const unsigned char* ss = sb + kDgBN * RB + 4 * r;  // the step's scales of row r
+      const float sc = axk::is_mx(F)   ? e8m0_to_f32(ss[2 * (ks & 1) + (g4 >> 1)])
+                       : axk::is_nv(F) ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(ss[g4], 1.0f, false)[0]
+                                       : 1.0f;
+      dg_decode<F>(sb + r * RB, g4, r, sc, bf[j]);
+    }
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) {
-      axk_bf16x8 af[kDgMT], bf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = brow[j] + l16;
-        const float sc = axk::is_mx(F)   ? e8m0_to_f32(sb[kDgBN * RB + 4 * r + 2 * (ks & 1) + kh])
-                         : axk::is_nv(F) ? e4m3_to_f32(sb[kDgBN * RB + 4 * r + 2 * kh + (g4 >> 1)])
-                                         : 1.0f;
-        bf[j] = dg_decode<F>(sb + r * RB, kh, g4, r, sc);
-      }
+      axk_bf16x8 af[kDgMT];
 #pragma unroll
       for (int mt = 0; mt < kDgMT; ++mt) {
         const int r = 16 * mt + l16;
-        af[mt] = *reinterpret_cast<const axk_bf16x8*>(sa + r * 128 + 16 * ((4 * kh + g4) ^ (r & 7)));
+        af[mt] = *reinterpret_cast<const axk_bf16x8*>(sa + r * 128 + 16 * ((2 * g4 + kh) ^ (r & 7)));
       }
 #pragma unroll
       for (int mt = 0; mt < kDgMT; ++mt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[mt][j] = mfma_bf16_16x16x32(af[mt], bf[j], acc[mt][j]);
+        for (int j = 0; j < 4; ++j) acc[mt][j] = mfma_bf16_16x16x32(af[mt], bf[j][kh], acc[mt][j]);
     }
   };
-  static_assert(kDgStages == 3, "the K loop is unrolled over three ring slots");
-  for (int ks = 0; ks < nk; ks += 3) {
-    step(ks, std::integral_constant<int, 0>{});
-    if (ks + 1 < nk) step(ks + 1, std::integral_constant<int, 1>{});
-    if (ks + 2 < nk) step(ks + 2, std::integral_constant<int, 2>{});
+  static_assert(ST == 3, "the K loop is unrolled over three ring slots (every LDS offset an immediate)");
+  // fp32 outputs of few rows are summed in eight runs of steps, the runs' sums apart, as the group kernel's eight waves
+  // sum them: one chain over K is further from the exact sum (248320 x 2048, 32 rows: 7.8e-8 of it against 5.6e-8)
+  constexpr bool kRuns = EPI == EPI_PLAIN && BM <= 64;
+  axk_f32x4 tot[kRuns ? kDgMT : 1][4];
+  auto end_run = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int mt = 0; mt < kDgMT; ++mt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        tot[mt][j] += acc[mt][j];
+        acc[mt][j] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  if constexpr (kRuns)
+#pragma unroll
+    for (int mt = 0; mt < kDgMT; ++mt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) tot[mt][j] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
+  const int run = (nk / 3 + 7) / 8;
+  for (int ks = 0, left = run; ks < nk; ks += 3) {
+    step(ks, 0);
+    if (ks + 1 < nk) step(ks + 1, 1);
+    if (ks + 2 < nk) step(ks + 2, 2);
+    if constexpr (kRuns)
+      if (g.out_f32 && --left == 0) {
+        end_run();
+        left = run;
+      }
+  }
+  if constexpr (kRuns) {
+#pragma unroll
+    for (int mt = 0; mt < kDgMT; ++mt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[mt][j] += tot[mt][j];
   }
   wait_vmcnt<0>();  // the look-ahead loads land before the workgroup's LDS is released
 
@@ -616,7 +647,7 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
   // bf16 outputs go through an LDS tile [BM rows][COLS + 8] over the ring, then leave as 16-byte row segments
   // (EPI_RES: the residual read the same way and added as bf16(res + bf16(v)))
   constexpr int LDO = COLS + 8;
-  static_assert(kDgBM * LDO * 2 <= kDgStages * STAGE, "the output tile fits in the ring");
+  static_assert(kDgBM * LDO * 2 <= ST * STAGE, "the output tile fits in the ring");
   uint16_t* so = reinterpret_cast<uint16_t*>(smem);
   __syncthreads();  // every wave is done with the ring
 #pragma unroll
@@ -676,16 +707,42 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
   }
 }
 
+// Column blocks of a group.
+inline int64_t dg_blocks(const MxGroup& g, int epi) {
+  if (epi == EPI_SWIGLU) return (g.n[0] + kDgBN / 2 - 1) / (kDgBN / 2);
+  int64_t nb = 0;
+  for (int i = 0; i < g.count; ++i) nb += (g.n[i] + kDgBN - 1) / kDgBN;
+  return nb;
+}
+
+// Where the dense GEMM is faster than the group kernel below 128 rows. The group kernel streams the weights once per 32
+// rows in many short workgroups, each reading its rows' whole activation; the GEMM once per call, in column blocks of
+// 256 whose K steps are a latency chain (0.5 us a step), so it needs enough of them. Measured (group kernel -> GEMM,
+// us; N x K, rows):
+//   MXFP4  24576 x 4096: 32 rows 41.3 -> 34.7;  16384 x 4096: 32 rows 28.1 -> 33.6, 64 rows 54.5 -> 33.7;
+//          8192 x 2048: 64 rows 19.4 -> 16.4, 100 rows 31.1 -> 17.2;  248320 x 2048: 32 rows 239 -> 87
+//   NVFP4  24576 x 4096: 32 rows 43.8 -> 41.9;  16384 x 4096: 64 rows 57.7 -> 41.9;  8192 x 2048: 64 rows 19.9 -> 24.2,
+//          100 rows 32.4 -> 24.5
+//   MXFP8  32768 x 4096: 32 rows 52.4 -> 63.0;  248320 x 2048: 32 rows 216 -> 117;  8192 x 2048: 64 rows 20.8 -> 18.5,
+//          100 rows 32.5 -> 18.5
+template <int F>
+bool dg_rows(int64_t m, int64_t blocks) {
+  if (m >= kDgMinRows) return true;
+  if (m <= 16) return false;
+  if (m <= 32) return blocks >= (axk::is_fp4(F) ? 96 : 192);
+  return blocks >= (axk::is_nv(F) && m <= 64 ? 64 : 32);
+}
+
 // The dense GEMM for a checked group: one launch for all of its matrices (their column blocks end to end; EPI_SWIGLU
 // the gate / up pair). dg_fits is false when the shape does not take it (then the group kernel runs).
 // MX formats load each step's E8M0 bytes as 4-byte aligned dwords of the scale rows: K a multiple of 128 (whole
 // dwords per row) and 4-byte aligned scale matrices.
 template <int F>
-bool dg_fits(int64_t m, int64_t k, const AxkConvEpi* conv, const MxGroup& g) {
+bool dg_fits(int64_t m, int64_t k, const AxkConvEpi* conv, const MxGroup& g, int epi) {
   if constexpr (F == axk::WF_BF16) {
     return false;
   } else {
-    if (conv != nullptr || m < kDgMinRows || k % kDgBK != 0 || dg_lds_bytes<F>(k) > 160 * 1024) return false;
+    if (conv != nullptr || k % kDgBK != 0 || !dg_rows<F>(m, dg_blocks(g, epi))) return false;
     if constexpr (axk::is_mx(F)) {
       if (k % 128 != 0) return false;
       for (int i = 0; i < g.count; ++i)
@@ -699,18 +756,31 @@ bool dg_fits(int64_t m, int64_t k, const AxkConvEpi* conv, const MxGroup& g) {
   }
 }
 
-template <int F, int EPI>
-int dg_launch(const DgArgs& d, hipStream_t st) {
+template <int F, int EPI, int BM>
+int dg_launch(const DgArgs& d, int64_t nb, hipStream_t st) {
   static AxkOnce lds_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
-  if (const int rc = axk_raise_lds(lds_once, reinterpret_cast<const void*>(&mx_gemm_kernel<F, EPI>), 160 * 1024))
+  if (const int rc = axk_raise_lds(lds_once, reinterpret_cast<const void*>(&mx_gemm_kernel<F, EPI, BM>), 160 * 1024))
     return rc;
-  constexpr int COLS = EPI == EPI_SWIGLU ? kDgBN / 2 : kDgBN;
-  const int64_t nb = EPI == EPI_PLAIN ? d.cb0[d.count] : ((int64_t)d.n[0] + COLS - 1) / COLS;
-  const int64_t tiles = nb * (((int64_t)d.m + dg_bm<F>() - 1) / dg_bm<F>());
+  const int64_t tiles = nb * (((int64_t)d.m + BM - 1) / BM);
   const int64_t grid = (tiles + kDgXcds - 1) / kDgXcds * kDgXcds;  // whole rounds over the XCDs
   AXK_REQUIRE(grid <= INT32_MAX, AXK_E_SHAPE);
-  hipLaunchKernelGGL((mx_gemm_kernel<F, EPI>), dim3((unsigned)grid), dim3(256), dg_lds_bytes<F>(d.k), st, d);
+  hipLaunchKernelGGL((mx_gemm_kernel<F, EPI, BM>), dim3((unsigned)grid), dim3(256), (dg_lds_bytes<F, BM>()), st, d);
   return axk_launch_status();
+}
+
+// Rows per workgroup: the most (each decoded weight fragment feeds BM / 16 MFMAs) that still gives every CU a workgroup.
+// 256 rows, MXFP4: [4096, 4096] 71.4 -> 40.0 us, [16384, 4096] 72.5 -> 51.2 (128-row workgroups before); a deeper ring
+// for calls of at most one workgroup a CU changed nothing (each step is bound by its own chain: barrier, LDS reads,
+// decode, MFMAs).
+template <int F, int EPI>
+int dg_epi(const DgArgs& d, hipStream_t st) {
+  constexpr int COLS = EPI == EPI_SWIGLU ? kDgBN / 2 : kDgBN;
+  const int64_t nb = EPI == EPI_PLAIN ? d.cb0[d.count] : ((int64_t)d.n[0] + COLS - 1) / COLS;
+  auto fills = [&](int bm) { return d.m > bm / 2 && nb * ((d.m + bm - 1) / bm) >= kDgCus; };
+  if constexpr (dg_bm<F>() > 64)
+    if (fills(dg_bm<F>())) return dg_launch<F, EPI, dg_bm<F>()>(d, nb, st);
+  if (fills(64)) return dg_launch<F, EPI, 64>(d, nb, st);
+  return dg_launch<F, EPI, 32>(d, nb, st);
 }
 
 template <int F>
@@ -731,9 +801,9 @@ int dg_group(const uint16_t* a, int64_t lda, const MxGroup& g, int epi, int64_t 
   d.ldr = g.ldr;
   d.out_f32 = g.out_f32;
   d.m = (int)m, d.k = (int)k;
-  if (epi == EPI_SWIGLU) return dg_launch<F, EPI_SWIGLU>(d, st);
-  if (epi == EPI_RES) return dg_launch<F, EPI_RES>(d, st);
-  return dg_launch<F, EPI_PLAIN>(d, st);  // every matrix of the group in one launch
+  if (epi == EPI_SWIGLU) return dg_epi<F, EPI_SWIGLU>(d, st);
+  if (epi == EPI_RES) return dg_epi<F, EPI_RES>(d, st);
+  return dg_epi<F, EPI_PLAIN>(d, st);  // every matrix of the group in one launch
 }
 
 // Checks a group and launches it. Matrices need whole 128-byte row segments (and 8-byte aligned MXFP4 scale rows).
@@ -804,7 +874,7 @@ int mx_group(const uint16_t* a, int64_t lda, const AxkMxMat* mats, int count, in
   for (int i = count; i <= AXK_MX_GROUP_MAX; ++i) g.tile0[i] = (int)tiles;
   if (m == 0) return AXK_OK;
   AXK_LAUNCH_GATE();
-  if (dg_fits<F>(m, k, conv, g)) return dg_group<F>(a, lda, g, epi, m, k, st);
+  if (dg_fits<F>(m, k, conv, g, epi)) return dg_group<F>(a, lda, g, epi, m, k, st);
   if (epi == EPI_SWIGLU) return group_dispatch<F, EPI_SWIGLU>(a, lda, g, m, k, st);
   if (epi == EPI_RES) return group_dispatch<F, EPI_RES>(a, lda, g, m, k, st);
   return group_dispatch<F, EPI_PLAIN>(a, lda, g, m, k, st);

@@ -1,0 +1,70 @@
+"""GPU parity of the runtime-weight linears at 17 .. 127 rows of wide matrices, where the dense GEMM takes over from the
+group kernel: both sides of each threshold, every tile of rows (32, 64, 128) at its edges, ragged channel counts, and a
+decode layer whose MLP takes the SwiGLU form. Bars as tests/test_gpu_linear_prefill.py."""
+import pytest
+import torch
+
+import axk
+from axk import configs, layer
+from oracle import layer as olayer
+from oracle import mx
+from test_gpu_linear_prefill import _close
+
+pytestmark = pytest.mark.gpu
+FUSED_TOL = dict(rtol=5e-2, atol=0.0625)
+
+
+def _run(fmt, m, n, k, out_dtype, dev):
+    g = torch.Generator().manual_seed(m * 7 + n + k)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    bias = torch.randn(n, generator=g) / 8
+    rb = bias.to(out_dtype).float()
+    kw = dict(out_dtype=out_dtype, bias=bias.to(dev))
+    if fmt == "mxfp4":
+        w, s = configs.mxfp4_weight(n, k, g)
+        return a, axk.mxfp4_gemm(a.to(dev), w.to(dev), s.to(dev), **kw), rb, mx.dequant_mxfp4(w.numpy(), s.numpy())
+    if fmt == "nvfp4":
+        w = configs.pack_codes(torch.randint(0, 16, (n, k), generator=g, dtype=torch.uint8))
+        s = torch.randint(0x28, 0x38, (n, k // 16), generator=g, dtype=torch.uint8)
+        got = axk.nvfp4_gemm(a.to(dev), w.to(dev), s.to(dev), torch.tensor([0.05], device=dev), **kw)
+        return a, got, rb, mx.dequant_nvfp4(w.numpy(), s.numpy(), 0.05)
+    if fmt == "fp8":
+        w, s = configs.fp8_proj_weight(n, k, g)
+        got = axk.fp8_gemm(a.to(dev), w.to(dev), None, s.to(dev), **kw)
+        return a, got, rb, mx.e4m3_table()[w.numpy()] * s.numpy()[:, None]
+    codes = torch.randint(0, 0x7B, (n, k), generator=g, dtype=torch.uint8)  # finite in both formats
+    s = torch.randint(119, 124, (n, k // 32), generator=g, dtype=torch.uint8)
+    if fmt == "e5m2":
+        codes = codes & 0x43  # magnitudes up to 3.5
+    return a, axk.mxfp8_gemm(a.to(dev), codes.to(dev), s.to(dev), fmt=fmt, **kw), rb, mx.dequant_mxfp8(
+        codes.numpy(), s.numpy(), fmt)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp4", "nvfp4", "fp8", "e4m3", "e5m2"])
+@pytest.mark.parametrize("m,n,k", [(16, 8200, 256), (17, 24600, 256), (32, 24320, 128), (33, 8200, 256), (64, 7936, 128),
+                                   (64, 16390, 384), (65, 8000, 256), (127, 8200, 128), (128, 300, 256),
+                                   (40, 8200, 192)])
+def test_rows_of_wide_matrices(dev, fmt, m, n, k):
+    out_dtype = torch.float32 if m % 2 else torch.bfloat16
+    if fmt != "fp8" and k % 128:
+        k = 320  # a K of whole 64s but not of whole scale dwords (the group or the unstaged kernel)
+    print(f"{fmt} m={m} n={n} k={k} {out_dtype}", flush=True)
+    a, got, bias, w = _run(fmt, m, n, k, out_dtype, dev)
+    wt = torch.from_numpy(w).float()
+    _close(got, a.float() @ wt.T + bias, out_dtype, a, wt)
+
+
+@pytest.mark.parametrize("mlp_fmt", ["mxfp4", "mxfp8"])
+def test_layer_mlp_of_40_rows(dev, mlp_fmt):
+    """40 sequences, MLP width 4096: gate | up take the dense GEMM's SwiGLU form, the other projections the group's."""
+    g = torch.Generator().manual_seed(40)
+    h, f, nk, nv, b = 256, 4096, 2, 4, 40
+    w = configs.gdn_layer_weights(g, h, f, nk, nv, mlp_fmt=mlp_fmt)
+    x = torch.randn(b, h, generator=g).bfloat16()
+    st = torch.randn(b, nv, 128, 128, generator=g) * 0.02
+    cv = torch.randn(b, 3, 2 * nk * 128 + nv * 128, generator=g).bfloat16()
+    print(f"layer of 40 rows {mlp_fmt}", flush=True)
+    out, _, _ = layer.gdn_layer_decode(x.to(dev), {n: t.to(dev) for n, t in w.items()}, st.to(dev), cv.to(dev), nk, nv,
+                                       mlp_fmt=mlp_fmt)
+    ref = olayer.gdn_layer_decode(x, w, st, cv, nk, nv, mlp_fmt=mlp_fmt)[0]
+    torch.testing.assert_close(out.float().cpu(), ref.float(), **FUSED_TOL)
