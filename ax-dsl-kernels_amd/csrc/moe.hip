@@ -455,7 +455,10 @@ constexpr int kStageLd = 64 * kBatchChunks + 16;    // bytes per staged weight r
 constexpr int kWaveStageBytes = 32 * kStageLd;      // a wave's LDS tile: gate and up, 16 rows each
 constexpr int kStageLpr = 4 * kBatchChunks;         // staged loads: lanes per row segment,
 constexpr int kStageRpi = 64 / kStageLpr;           // rows per load instruction (kBatchChunks instructions a tile)
-constexpr int kSmallRows = 8;                       // activation rows per pass of the staged kernels
+// activation rows per pass of the staged kernels: 8 (gate-up: 51 KiB of LDS at H 2048, three workgroups a CU), or 12 (gate-up: 67
+// KiB, two) and kStageRows (down: 35 KiB at F 512) where the experts' rows would often take a second pass, which streams
+// the expert's weights again
+constexpr int kSmallRows = 8, kMidRows = 12;
 constexpr int kStreamThreads = 64 * kStreamWaves;
 // byte offset of the wave tiles after the activation rows ([rows][K + 8] bf16), 16-byte aligned
 __host__ __device__ inline size_t stream_stage_off(int rows, int K) { return ((size_t)rows * (K + 8) * 2 + 15) & ~(size_t)15; }
@@ -1329,26 +1332,31 @@ __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
     issue(ks + 2, (BUF + 2) % kGStages);  // into the slot of step ks - 1
     const unsigned char* sa = smem + BUF * STAGE;
     const unsigned char* sb = sa + kGAStage;
+    // a lane's 16 weights of the step, k = 16 g4 .. + 15 of the row: one LDS read and one block scale, the B operands of
+    // two MFMAs (MFMA kh takes k = 16 g4 + 8 kh + j for its index (g4, j), in both operands)
+    axk_bf16x8 bf[4][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = brow[j] + l16;
+      const uint2 w = *reinterpret_cast<const uint2*>(sb + r * 32 + 16 * ((g4 >> 1) ^ ((r >> 3) & 1)) + 8 * (g4 & 1));
+      const uint32_t sbyte =
+          SDMA ? sb[kGBStage + 4 * r + 2 * (ks & 1) + (g4 >> 1)] : sS[r * ldS + 2 * ks + (g4 >> 1)];
+      const float sc = e8m0_to_f32(sbyte);
+      bf[j][0] = fp4x8_to_bf16x8(w.x, sc);
+      bf[j][1] = fp4x8_to_bf16x8(w.y, sc);
+    }
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) {
-      axk_bf16x8 af[kGMT], bf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = brow[j] + l16;
-        const uint32_t w = *reinterpret_cast<const uint32_t*>(sb + r * 32 + 16 * (kh ^ ((r >> 3) & 1)) + 4 * g4);
-        // one E8M0 byte: two VALU to an fp32 scale
-        const uint32_t sbyte = SDMA ? sb[kGBStage + 4 * r + 2 * (ks & 1) + kh] : sS[r * ldS + 2 * ks + kh];
-        bf[j] = fp4x8_to_bf16x8(w, e8m0_to_f32(sbyte));
-      }
+      axk_bf16x8 af[kGMT];
 #pragma unroll
       for (int mt = 0; mt < kGMT; ++mt) {
         const int r = 16 * mt + l16;
-        af[mt] = *reinterpret_cast<const axk_bf16x8*>(sa + r * 128 + 16 * ((4 * kh + g4) ^ (r & 7)));
+        af[mt] = *reinterpret_cast<const axk_bf16x8*>(sa + r * 128 + 16 * ((2 * g4 + kh) ^ (r & 7)));
       }
 #pragma unroll
       for (int mt = 0; mt < kGMT; ++mt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[mt][j] = mfma_bf16_16x16x32(af[mt], bf[j], acc[mt][j]);
+        for (int j = 0; j < 4; ++j) acc[mt][j] = mfma_bf16_16x16x32(af[mt], bf[j][kh], acc[mt][j]);
     }
   };
   static_assert(kGStages == 3, "the K loop is unrolled over three ring slots");
@@ -1549,27 +1557,39 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   }
   const int max_slots = E < T * K ? E : T * K;
   const int fmax = F > Fs ? F : Fs;
-  // runs of 4 x tpw tiles per workgroup; activation rows staged in dynamic LDS ([rows][K + 8] bf16). Small batches
-  // (tokens <= 64, K a multiple of 256) take the staged-weight kernels with 8 activation rows per pass (their
-  // LDS tiles fit beside 8 rows, not 16); the others stream MFMA-layout units with 16 rows per pass.
+  // runs of 4 x tpw tiles per workgroup; activation rows staged in dynamic LDS ([rows][K + 8] bf16). Where K is a
+  // multiple of 256 the weights are staged through LDS as whole row segments, with 8, 12 or 16 activation rows per pass
+  // by how many rows an expert has on average (T K / E); the others stream MFMA-layout units with 16 rows per pass.
+  // Measured (E 256, top-8, H 2048, F 512; us at 65 / 100 / 150 / 200 / 256 tokens): unstaged 16 rows above 64 tokens
+  // 120 / 133 / 155 / 161 / 173; staged, gate-up 8 rows and down 8 99 / 114 / 138 / 163 / 189, gate-up 8 and down 16 102 / 114 /
+  // 138 / 155 / 173, gate-up 12 and down 16 112 / 122 / 142 / 150 / 166.
   const int gu_tpw = kGateUpTilesPerWave, dn_tpw = kDownTilesPerWave;
   const int run_gu = kStreamWaves * gu_tpw, run_dn = kStreamWaves * dn_tpw;
   const int gu_grp = ((fmax + 15) / 16 + run_gu - 1) / run_gu;
   const int dn_grp = ((H + 15) / 16 + run_dn - 1) / run_dn;
   const int wide_k = 128 * kBatchChunks;
   const bool gu_wide = H % wide_k == 0, dn_wide = F % wide_k == 0 && Fs % wide_k == 0;
-  const bool gu_stage = gu_wide && T <= 64, dn_stage = dn_wide && T <= 64;
-  const int gu_rows = gu_stage ? kSmallRows : kStageRows, dn_rows = dn_stage ? kSmallRows : kStageRows;
-  const size_t gu_lds = stream_stage_off(gu_rows, H) + (gu_stage ? kStreamWaves * kWaveStageBytes : 0);
-  const size_t dn_lds = stream_stage_off(dn_rows, fmax) + (dn_stage ? kStreamWaves * kWaveStageBytes : 0);
+  const size_t stage_lds = kStreamWaves * kWaveStageBytes;
+  const bool many = T > 64;  // (a size that 16 unstaged rows would not fit is refused there, staged or not)
+  AXK_REQUIRE(!many || (stream_stage_off(kStageRows, H) <= kMaxStreamLds &&
+                        stream_stage_off(kStageRows, fmax) <= kMaxStreamLds), AXK_E_SHAPE);
+  const bool gu_stage = gu_wide, dn_stage = dn_wide;
+  const bool gu_mid = gu_stage && many && (int64_t)T * K > 5 * (int64_t)E &&
+                      stream_stage_off(kMidRows, H) + stage_lds <= kMaxStreamLds;
+  const bool dn_full = dn_stage && many && (int64_t)T * K > 4 * (int64_t)E &&
+                       stream_stage_off(kStageRows, fmax) + stage_lds <= kMaxStreamLds;
+  const int gu_rows = gu_mid ? kMidRows : gu_stage ? kSmallRows : kStageRows;
+  const int dn_rows = dn_full || !dn_stage ? kStageRows : kSmallRows;
+  const size_t gu_lds = stream_stage_off(gu_rows, H) + (gu_stage ? stage_lds : 0);
+  const size_t dn_lds = stream_stage_off(dn_rows, fmax) + (dn_stage ? stage_lds : 0);
   AXK_REQUIRE(gu_lds <= kMaxStreamLds && dn_lds <= kMaxStreamLds, AXK_E_SHAPE);
   static AxkOnce lds_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
   const int raised = axk_once(lds_once, [] {
-    const void* fns[6] = {reinterpret_cast<const void*>(&moe_gateup_kernel<false, kStageRows, false>),
-                          reinterpret_cast<const void*>(&moe_gateup_kernel<true, kStageRows, false>),
+    const void* fns[6] = {reinterpret_cast<const void*>(&moe_gateup_kernel<true, kMidRows, true>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<true, kStageRows, true>),
+                          reinterpret_cast<const void*>(&moe_gateup_kernel<false, kStageRows, false>),
                           reinterpret_cast<const void*>(&moe_gateup_kernel<true, kSmallRows, true>),
                           reinterpret_cast<const void*>(&moe_down_kernel<false, kStageRows, false>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<true, kStageRows, false>),
                           reinterpret_cast<const void*>(&moe_down_kernel<true, kSmallRows, true>)};
     for (const void* f : fns) {
       const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxStreamLds);
@@ -1582,17 +1602,17 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   GateUpArgs ga{h2, e_gw, e_gs, sh_gate_w, sh_gate_s, sh_up_w, sh_up_s, topk_ids, T, H, F, Fs, E, K, gu_grp, gu_tpw,
                 gu_nsp, w};
   const dim3 gu_grid((unsigned)((max_slots + gu_nsp) * gu_grp)), dn_grid((unsigned)((max_slots + dn_nsp) * dn_grp));
-  if (gu_stage)
+  if (gu_mid)
+    hipLaunchKernelGGL((moe_gateup_kernel<true, kMidRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+  else if (gu_stage)
     hipLaunchKernelGGL((moe_gateup_kernel<true, kSmallRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
-  else if (gu_wide)
-    hipLaunchKernelGGL((moe_gateup_kernel<true, kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   else
     hipLaunchKernelGGL((moe_gateup_kernel<false, kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   DownArgs da{e_dw, e_ds, sh_down_w, sh_down_s, topk_ids, topk_weights, T, H, F, Fs, E, K, dn_grp, dn_tpw, dn_nsp, w};
-  if (dn_stage)
+  if (dn_full)
+    hipLaunchKernelGGL((moe_down_kernel<true, kStageRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+  else if (dn_stage)
     hipLaunchKernelGGL((moe_down_kernel<true, kSmallRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
-  else if (dn_wide)
-    hipLaunchKernelGGL((moe_down_kernel<true, kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   else
     hipLaunchKernelGGL((moe_down_kernel<false, kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   // the decode router formed the shared gate's logit when the routing ran in this call (gate_given)

@@ -1,0 +1,33 @@
+"""GPU parity of the MoE decode kernels above 64 tokens, where the activation rows per pass (8, 12 or 16) follow the rows an
+expert has: experts of one pass and of several, at the rows where the choice changes, with and without a shared expert of
+another width, and hidden or expert widths that are not whole batches (the unstaged kernels). Bars of
+tests/test_gpu_moe.py."""
+import pytest
+import torch
+
+from axk import configs
+from test_gpu_moe import _check_layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("t,h,e,f,fs,k", [
+    (65, 512, 32, 256, 256, 4),    # 8 rows an expert: gate-up 12, down 16
+    (65, 512, 64, 256, 512, 4),    # 4 rows: gate-up 8, down 8; a wider shared expert
+    (80, 256, 64, 512, 256, 4),    # 5 rows: gate-up 8, down 16
+    (81, 256, 64, 512, 0, 4),      # past 5: gate-up 12; no shared expert
+    (256, 256, 8, 256, 256, 2),    # 64 rows an expert: several passes of each
+    (200, 512, 300, 256, 256, 2),  # 1.3 rows: single passes, more than 256 experts
+    (100, 512, 16, 96, 160, 3),    # staged gate-up, unstaged down
+    (100, 384, 16, 256, 256, 3),   # unstaged gate-up, staged down
+])
+def test_rows_per_pass(dev, t, h, e, f, fs, k):
+    g = torch.Generator().manual_seed(t + h + e)
+    w = configs.moe_weights(g, hidden=h, experts=e, inter=f, shared_inter=max(fs, 32), router_std=0.5)
+    if fs == 0:
+        for n in ("w_gate", "s_gate", "w_up", "s_up", "w_down", "s_down", "w_shg"):
+            w.pop(n)
+    c = {"h2": torch.randn(t, h, generator=g).to(torch.bfloat16),
+         "x_res": torch.randn(t, h, generator=g).to(torch.bfloat16), "weights": w, "top_k": k}
+    print(f"case t={t} h={h} e={e} f={f} fs={fs} k={k}", flush=True)
+    _check_layer(c, dev)
