@@ -58,7 +58,18 @@ constexpr int kDecodeTokens = 64 * kMaskWords;  // above this the prefill path r
 constexpr int64_t kMaxPrefillTokens = 1 << 16;
 constexpr int64_t kMaxPrefillPairs = 1 << 19;
 constexpr int kBlkTokens = 256;  // tokens per block of the prefill grouping
-constexpr int kBM = 128, kBK = 64;  // prefill GEMM tile rows, K step
+constexpr int kBM = 128, kBK = 64;  // prefill GEMM: most rows of a tile, K step
+// The rows of a tile: 32 or 64 where the experts' rows are few on average (T K / E), so that the GEMMs neither load nor
+// multiply tiles that are mostly padding. Measured (E 256, top-8, H 2048, F 512; us with 32- / 64- / 128-row tiles):
+// 257 tokens 182 / 193 / 216, 700 tokens 196 / 206 / 227, 1024 tokens 227 / 216 / 236, 1400 tokens 266 / 227 / 246,
+// 2048 tokens 320 / 273 / 272, 4096 tokens 544 / 428 / 408. Around 128 rows an expert, half the experts have a few more
+// than a 128-row tile takes, and their second tiles stream and decode the weights again: 160-row tiles there (4096
+// tokens 426 -> 397 us on one box; 2800 tokens, whose experts fit 128 rows, 328 -> 348).
+constexpr int kBMWide = 160;
+inline int tile_rows(int64_t T, int64_t E, int64_t K) {
+  const int64_t p = T * K;
+  return p <= 26 * E ? 32 : p <= 56 * E ? 64 : p > 120 * E && p <= 165 * E ? kBMWide : kBM;
+}
 
 struct MoeWs {
   int* counts;      // [E]
@@ -84,7 +95,8 @@ struct MoeWs {
 
 int64_t prefill_blocks(int64_t T) { return (T + kBlkTokens - 1) / kBlkTokens; }
 int64_t prefill_max_tiles(int64_t T, int64_t E, int64_t K) {
-  return (T * K + kBM - 1) / kBM + E + (T + kBM - 1) / kBM;
+  const int64_t tb = tile_rows(T, E, K);
+  return (T * K + tb - 1) / tb + E + (T + tb - 1) / tb;
 }
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -103,7 +115,7 @@ constexpr int kWsParts = 17;
 size_t moe_ws_layout(int64_t T, int64_t H, int64_t E, int64_t K, int64_t F, int64_t Fs, size_t* off) {
   const int64_t P = T * K;
   const bool prefill = T > kDecodeTokens;
-  const size_t nb = prefill ? (size_t)prefill_blocks(T) : 0, nt = prefill ? (size_t)prefill_max_tiles(T, E, K) : 0;
+  const size_t nb = prefill ? (size_t)prefill_blocks(T) : 0, nt = prefill ? (size_t)((P + kBM - 1) / kBM + E + (T + kBM - 1) / kBM) : 0;
   const size_t S = prefill ? kPrefillRouterSplits : router_splits(H);
   const size_t rp = S * T * E * 4;
   size_t o = 0;
@@ -123,13 +135,16 @@ MoeWs moe_ws(void* ws, int64_t T, int64_t H, int64_t E, int64_t K, int64_t F, in
   size_t off[kWsParts];
   moe_ws_layout(T, H, E, K, F, Fs, off);
   unsigned char* b = reinterpret_cast<unsigned char*>(ws);
+  // a list of 32- or 64-row tiles, longer than its part, takes the half of y that bf16 rows leave (T K H bytes a half,
+  // the list at most T K / 2 + 16 E + T / 2 + 48)
+  const size_t tiles = T > kDecodeTokens && tile_rows(T, E, K) < kBM ? off[9] + (size_t)T * K * H * 2 : off[12];
   return {reinterpret_cast<int*>(b + off[0]),       reinterpret_cast<int*>(b + off[1]),
           reinterpret_cast<int4*>(b + off[2]),      reinterpret_cast<int*>(b + off[3]),
           reinterpret_cast<int*>(b + off[4]),       reinterpret_cast<int*>(b + off[5]),
           reinterpret_cast<float*>(b + off[6]),     reinterpret_cast<uint16_t*>(b + off[7]),
           reinterpret_cast<uint16_t*>(b + off[8]),  reinterpret_cast<float*>(b + off[9]),
           reinterpret_cast<float*>(b + off[10]),    reinterpret_cast<int*>(b + off[11]),
-          reinterpret_cast<int4*>(b + off[12]),     reinterpret_cast<int*>(b + off[13]),
+          reinterpret_cast<int4*>(b + tiles),      reinterpret_cast<int*>(b + off[13]),
           reinterpret_cast<int*>(b + off[14]),      reinterpret_cast<float*>(b + off[15]),
           reinterpret_cast<float*>(b + off[16]),    reinterpret_cast<float*>(b + off[16]) + T};
 }
@@ -1049,7 +1064,7 @@ __global__ __launch_bounds__(256) void moe_pcount_kernel(const int32_t* __restri
 
 // One workgroup: expert totals, offsets and active list; per-(block, expert) row bases (in place of the
 // counts); the GEMM tile list (routed experts in expert order, then the shared expert's tiles).
-__global__ __launch_bounds__(256) void moe_pscan_kernel(int T, int E, int NB, int has_shared, MoeWs w) {
+__global__ __launch_bounds__(256) void moe_pscan_kernel(int T, int E, int NB, int has_shared, int tb, MoeWs w) {
   __shared__ int s_tmp[12];
   constexpr int EPT = kMaxExperts / 256;
   const int tid = threadIdx.x;
@@ -1077,7 +1092,7 @@ __global__ __launch_bounds__(256) void moe_pscan_kernel(int T, int E, int NB, in
   for (int j = 0; j < EPT; ++j) {
     sum += cnt[j];
     nact += cnt[j] > 0;
-    ntile += (cnt[j] + kBM - 1) / kBM;
+    ntile += (cnt[j] + tb - 1) / tb;
   }
   int tot, tota, tott;
   int off = block_exclusive_scan256(sum, s_tmp, &tot);
@@ -1121,12 +1136,12 @@ __global__ __launch_bounds__(256) void moe_pscan_kernel(int T, int E, int NB, in
         w.active[aoff] = make_int4(cnt[j], e, off, 0);
         ++aoff;
       }
-      for (int r = 0; r < cnt[j]; r += kBM) w.tiles[toff++] = make_int4(e, off + r, min(kBM, cnt[j] - r), 0);
+      for (int r = 0; r < cnt[j]; r += tb) w.tiles[toff++] = make_int4(e, off + r, min(tb, cnt[j] - r), 0);
     }
     off += cnt[j];
   }
-  const int nsh = has_shared ? (T + kBM - 1) / kBM : 0;
-  for (int i = tid; i < nsh; i += blockDim.x) w.tiles[tott + i] = make_int4(-1, i * kBM, min(kBM, T - i * kBM), 0);
+  const int nsh = has_shared ? (T + tb - 1) / tb : 0;
+  for (int i = tid; i < nsh; i += blockDim.x) w.tiles[tott + i] = make_int4(-1, i * tb, min(tb, T - i * tb), 0);
   if (tid == 0) {
     w.offsets[E] = tot;
     *w.n_active = tota;
@@ -1186,27 +1201,32 @@ constexpr int kG2Rows = 256;          // weight rows per workgroup
 constexpr int kG2Cols0 = kG2Rows / 2;  // gate-up: output (act) columns per workgroup
 constexpr int kG2Cols1 = kG2Rows;      // down: output columns per workgroup
 constexpr int kXcds = 8;              // MI355X: consecutive workgroups go round-robin over 8 XCDs
-constexpr int kGStages = 3;
-// rows per workgroup: the gate-up GEMM takes a whole kBM-row tile (each decoded weight fragment feeds 8 MFMAs); the
-// down GEMM (K = F, a short reduction) a half tile, so twice the workgroups share its fixed costs
-template <int MODE>
-constexpr int g_bm() { return MODE == 0 ? kBM : kBM / 2; }
-template <int MODE>
-constexpr int g_astage() { return g_bm<MODE>() * kBK * 2; }
+// rows per workgroup of a TB-row tile: the gate-up GEMM takes the whole tile (each decoded weight fragment feeds TB / 16
+// MFMAs); of a 128-row tile the down GEMM (K = F, a short reduction) takes half, so twice the workgroups share its
+// fixed costs (a 160-row tile: 64, 64 and 32)
+template <int MODE, int TB>
+constexpr int g_bm() { return MODE == 1 && TB > 64 ? 64 : TB; }
+// ring slots: two for the 160-row gate-up tile (59 KiB, two workgroups a CU; a step's arithmetic covers the next step's
+// loads), else three
+template <int MODE, int TB>
+constexpr int g_stages() { return MODE == 0 && TB > kBM ? 2 : 3; }
+template <int MODE, int TB>
+constexpr int g_astage() { return g_bm<MODE, TB>() * kBK * 2; }
 constexpr int kGBStage = kG2Rows * kBK / 2;  // 8 KiB
-template <int MODE>
-constexpr int g_stage() { return g_astage<MODE>() + kGBStage; }
+template <int MODE, int TB>
+constexpr int g_stage() { return g_astage<MODE, TB>() + kGBStage; }
 constexpr int kGSStage = kG2Rows * 4;  // SDMA: one scale dword per weight row and step
-template <int MODE>
+template <int MODE, int TB>
 size_t gemm_lds_bytes(int Kd, bool sdma) {
-  return sdma ? (size_t)kGStages * (g_stage<MODE>() + kGSStage)
-              : (size_t)kGStages * g_stage<MODE>() + (size_t)kG2Rows * (Kd / 32 + 16);
+  return sdma ? (size_t)g_stages<MODE, TB>() * (g_stage<MODE, TB>() + kGSStage)
+              : (size_t)g_stages<MODE, TB>() * g_stage<MODE, TB>() + (size_t)kG2Rows * (Kd / 32 + 16);
 }
 
-template <int MODE, bool SDMA>
+template <int MODE, bool SDMA, int TB>
 __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
-  constexpr int BM = g_bm<MODE>(), SUB = kBM / BM;              // rows per workgroup, workgroups per tile
-  constexpr int kGAStage = g_astage<MODE>(), kGStage = g_stage<MODE>();
+  constexpr int BM = g_bm<MODE, TB>(), SUB = (TB + BM - 1) / BM;  // rows per workgroup, workgroups per tile
+  constexpr int kGStages = g_stages<MODE, TB>();
+  constexpr int kGAStage = g_astage<MODE, TB>(), kGStage = g_stage<MODE, TB>();
   constexpr int kGAI = kGAStage / 1024 / 4;                        // A direct-load instructions per wave and step
   constexpr int kGMT = BM / 16;                                    // 16-row MFMA tiles per wave (all rows of the tile)
   constexpr int STAGE = kGStage + (SDMA ? kGSStage : 0);
@@ -1289,8 +1309,8 @@ __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
     for (int h = 0; h < 2; ++h) lds_dma16_cached(bsrc[h] + kk * (kBK / 2), base + kGAStage + (2 * wave + h) * 1024);
     if constexpr (SDMA) lds_dma4_cached(ssrc + 4 * (kk >> 1), base + kGStage + 256 * wave);
   };
-  issue(0, 0);
-  issue(1, 1);
+#pragma unroll
+  for (int i = 0; i < kGStages - 1; ++i) issue(i, i);
 
   // the E8M0 scales of the whole reduction (while the first steps load): 16-byte units when the row length
   // allows, else 2-byte units
@@ -1325,11 +1345,12 @@ __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
   // step ks from ring slot BUF (a constant: the loop is unrolled over the ring, so every LDS offset is immediate)
   auto step = [&](int ks, auto buf_c) __attribute__((always_inline)) {
     constexpr int BUF = decltype(buf_c)::value;
-    wait_vmcnt<kGAI + 2 + (SDMA ? 1 : 0)>();  // this wave's loads of step ks have landed (step ks + 1's may not)
+    // this wave's loads of step ks have landed (with three slots step ks + 1's may not)
+    wait_vmcnt<(kGStages - 2) * (kGAI + 2 + (SDMA ? 1 : 0))>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of step ks - 1 are done
     __builtin_amdgcn_s_barrier();  // every wave's step-ks loads landed; every wave is done with step ks - 1
     asm volatile("" ::: "memory");
-    issue(ks + 2, (BUF + 2) % kGStages);  // into the slot of step ks - 1
+    issue(ks + kGStages - 1, (BUF + kGStages - 1) % kGStages);  // into the slot of step ks - 1
     const unsigned char* sa = smem + BUF * STAGE;
     const unsigned char* sb = sa + kGAStage;
     // a lane's 16 weights of the step, k = 16 g4 .. + 15 of the row: one LDS read and one block scale, the B operands of
@@ -1359,11 +1380,11 @@ __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
         for (int j = 0; j < 4; ++j) acc[mt][j] = mfma_bf16_16x16x32(af[mt], bf[j][kh], acc[mt][j]);
     }
   };
-  static_assert(kGStages == 3, "the K loop is unrolled over three ring slots");
-  for (int ks = 0; ks < nk; ks += 3) {
+  for (int ks = 0; ks < nk; ks += kGStages) {
     step(ks, std::integral_constant<int, 0>{});
     if (ks + 1 < nk) step(ks + 1, std::integral_constant<int, 1>{});
-    if (ks + 2 < nk) step(ks + 2, std::integral_constant<int, 2>{});
+    if constexpr (kGStages == 3)
+      if (ks + 2 < nk) step(ks + 2, std::integral_constant<int, 2>{});
   }
   wait_vmcnt<0>();  // the look-ahead loads land before the workgroup's LDS is released
 
@@ -1372,6 +1393,7 @@ __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
   // 2-byte stores of 16 lanes; the shared expert's fp32 down rows are stored directly.
   constexpr int COLS = MODE == 0 ? kG2Cols0 : kG2Cols1, LDO = COLS + 8;
   const bool staged = MODE == 0 || !shared;
+  static_assert(BM * LDO * 2 <= kGStages * kGStage && BM * (COLS / 8) % 256 == 0, "the output tile fits in the ring");
   uint16_t* so = reinterpret_cast<uint16_t*>(smem);
   if (staged) __syncthreads();  // every wave is done with the ring
 #pragma unroll
@@ -1427,6 +1449,28 @@ __global__ __launch_bounds__(256, 2) void moe_ggemm_kernel(GGemmArgs g) {
       for (int e = 0; e < 8 && col + e < No; ++e) dst[e] = src[e];
     }
   }
+}
+
+template <int MODE, int TB>
+int launch_ggemm(const GGemmArgs& g, bool sdma, unsigned wgs, int Kd, hipStream_t st) {
+  static AxkOnce once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
+  const int raised = axk_once(once, [] {
+    const void* fns[2] = {reinterpret_cast<const void*>(&moe_ggemm_kernel<MODE, false, TB>),
+                          reinterpret_cast<const void*>(&moe_ggemm_kernel<MODE, true, TB>)};
+    for (const void* f : fns) {
+      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxStageLds);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  });
+  if (raised != AXK_OK) return raised;
+  const size_t lds = gemm_lds_bytes<MODE, TB>(Kd, sdma);
+  const dim3 grid((wgs + kXcds - 1) / kXcds * kXcds);  // whole rounds over the XCDs
+  if (sdma)
+    hipLaunchKernelGGL((moe_ggemm_kernel<MODE, true, TB>), grid, dim3(256), lds, st, g);
+  else
+    hipLaunchKernelGGL((moe_ggemm_kernel<MODE, false, TB>), grid, dim3(256), lds, st, g);
+  return axk_launch_status();
 }
 
 struct MoeDims {
@@ -1513,10 +1557,10 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   const int combine_shared = (has_shared || y_sh_given) ? 1 : 0;
   const int T = (int)tokens, H = (int)hidden, E = (int)num_experts, K = (int)top_k, F = (int)inter, Fs = (int)d.Fs;
   if (T > kDecodeTokens) {
-    const int NB = (int)prefill_blocks(T);
+    const int NB = (int)prefill_blocks(T), tb = tile_rows(T, E, K);
     // the (block, expert) counts: counted by the routing launch when it ran in this call, else from the ids
     if (!counted) hipLaunchKernelGGL(moe_pcount_kernel, dim3((unsigned)NB), dim3(256), 0, st, topk_ids, T, E, K, w);
-    hipLaunchKernelGGL(moe_pscan_kernel, dim3(1), dim3(256), 0, st, T, E, NB, has_shared ? 1 : 0, w);
+    hipLaunchKernelGGL(moe_pscan_kernel, dim3(1), dim3(256), 0, st, T, E, NB, has_shared ? 1 : 0, tb, w);
     hipLaunchKernelGGL(moe_pscatter_kernel, dim3((unsigned)NB), dim3(256), 0, st, topk_ids, topk_weights, T, E, K, w);
     const unsigned tiles = (unsigned)prefill_max_tiles(T, E, K);
     const int fmax = F > Fs ? F : Fs;
@@ -1525,32 +1569,19 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
     auto a4 = [](const void* p) { return p == nullptr || axk_aligned(p, 4); };
     const bool sdma0 = H % 128 == 0 && a4(e_gs) && a4(sh_gate_s) && a4(sh_up_s);
     const bool sdma1 = F % 128 == 0 && Fs % 128 == 0 && a4(e_ds) && a4(sh_down_s);
-    const size_t lds0 = gemm_lds_bytes<0>(H, sdma0), lds1 = gemm_lds_bytes<1>(fmax, sdma1);
-    static AxkOnce gemm_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
-    const int raised = axk_once(gemm_once, [] {
-      const void* fns[4] = {reinterpret_cast<const void*>(&moe_ggemm_kernel<0, false>),
-                            reinterpret_cast<const void*>(&moe_ggemm_kernel<1, false>),
-                            reinterpret_cast<const void*>(&moe_ggemm_kernel<0, true>),
-                            reinterpret_cast<const void*>(&moe_ggemm_kernel<1, true>)};
-      for (const void* f : fns) {
-        const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxStageLds);
-        if (e != hipSuccess) return e;
-      }
-      return hipSuccess;
-    });
-    if (raised != AXK_OK) return raised;
     const unsigned nb0 = (unsigned)((fmax + kG2Cols0 - 1) / kG2Cols0), nb1 = (unsigned)((H + kG2Cols1 - 1) / kG2Cols1);
-    auto xgrid = [](unsigned n) { return dim3((n + kXcds - 1) / kXcds * kXcds); };  // whole rounds over the XCDs
-    if (sdma0)
-      hipLaunchKernelGGL((moe_ggemm_kernel<0, true>), xgrid(tiles * nb0), dim3(256), lds0, st, gu);
-    else
-      hipLaunchKernelGGL((moe_ggemm_kernel<0, false>), xgrid(tiles * nb0), dim3(256), lds0, st, gu);
     GGemmArgs dn{w.act, w.act_sh, e_dw, e_ds, sh_down_w, sh_down_s, nullptr, nullptr, T, H, F, Fs, fmax, w};
-    constexpr unsigned sub1 = kBM / g_bm<1>();  // down workgroups per tile
-    if (sdma1)
-      hipLaunchKernelGGL((moe_ggemm_kernel<1, true>), xgrid(tiles * sub1 * nb1), dim3(256), lds1, st, dn);
-    else
-      hipLaunchKernelGGL((moe_ggemm_kernel<1, false>), xgrid(tiles * sub1 * nb1), dim3(256), lds1, st, dn);
+    int rc2;
+    if (tb == 32) rc2 = launch_ggemm<0, 32>(gu, sdma0, tiles * nb0, H, st);
+    else if (tb == 64) rc2 = launch_ggemm<0, 64>(gu, sdma0, tiles * nb0, H, st);
+    else if (tb == kBM) rc2 = launch_ggemm<0, kBM>(gu, sdma0, tiles * nb0, H, st);
+    else rc2 = launch_ggemm<0, kBMWide>(gu, sdma0, tiles * nb0, H, st);
+    if (rc2 != AXK_OK) return rc2;
+    if (tb == 32) rc2 = launch_ggemm<1, 32>(dn, sdma1, tiles * nb1, fmax, st);
+    else if (tb == 64) rc2 = launch_ggemm<1, 64>(dn, sdma1, tiles * nb1, fmax, st);
+    else if (tb == kBM) rc2 = launch_ggemm<1, kBM>(dn, sdma1, tiles * 2 * nb1, fmax, st);
+    else rc2 = launch_ggemm<1, kBMWide>(dn, sdma1, tiles * 3 * nb1, fmax, st);
+    if (rc2 != AXK_OK) return rc2;
     CombineArgs ca{h2, x_res, w_shg, nullptr, topk_ids, combine_shared, T, H, E, K, w, out};
     launch_combine<true>(ca, st);
     return axk_launch_status();

@@ -31,3 +31,18 @@ def test_rows_per_pass(dev, t, h, e, f, fs, k):
          "x_res": torch.randn(t, h, generator=g).to(torch.bfloat16), "weights": w, "top_k": k}
     print(f"case t={t} h={h} e={e} f={f} fs={fs} k={k}", flush=True)
     _check_layer(c, dev)
+
+
+@pytest.mark.parametrize("t,h,e,f,fs,k", [
+    (257, 256, 64, 128, 128, 2),   # 8 rows an expert: 32-row tiles
+    (260, 256, 20, 128, 128, 2),   # 26 rows: 32-row tiles, some experts over one
+    (280, 256, 20, 64, 64, 2),     # past 26 (28): 64-row tiles, widths without whole scale dwords
+    (280, 256, 10, 192, 0, 2),     # 56 rows: the last of the 64-row tiles, no shared expert
+    (300, 192, 10, 128, 128, 2),   # past 56: 128-row tiles
+    (305, 256, 5, 128, 128, 2),    # 122 rows: 160-row tiles
+    (330, 128, 4, 192, 64, 2),     # 165 rows: 160-row tiles, most experts over one
+    (340, 256, 4, 128, 128, 2),    # 170: 128-row tiles again
+    (300, 256, 2, 128, 128, 1),    # one expert near 150, top-1
+])
+def test_prefill_tile_rows(dev, t, h, e, f, fs, k):
+    test_rows_per_pass(dev, t, h, e, f, fs, k)
