@@ -1143,7 +1143,7 @@ __global__ __launch_bounds__(256) void paged_kv_write_fp8_kernel(const uint16_t*
 //
 // What bounds it: one wave issues at most one instruction every four cycles, and a pair's 32 MFMAs (1024 cycles)
 // bring about 300 others. Measured at D = 256, HQ 16, HKV 2: a 4096-token chunk 178 us, 773 TFLOP/s (237 us with 16
-// rows a wave, 16x16x32 MFMA and two waves a SIMD); 256 tokens after 16000 cached ones 96 us with the KV splits
+// rows a wave, 16x16x32 MFMA and two waves a SIMD); 256 tokens after 16000 cached ones 98 us with the KV splits
 // (814 us before: 32 row blocks on 256 CUs).
 typedef short axk_s16x8 __attribute__((ext_vector_type(8)));
 typedef float axk_f32x16 __attribute__((ext_vector_type(16)));
@@ -1327,20 +1327,25 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
   // lane l holds the address of page 64 chunk + l of the sequence (this KV head, this wave's plane); bad: the lanes
   // whose page is outside the pool (they hold page 0's)
   const unsigned char* const head0 = cache + (int64_t)kvh * D * 2 + plane * plane_stride;
-  int chunk = (t_beg / tpp) >> 6;
+  int chunk = 0;
   uint32_t pg_lo, pg_hi;
   unsigned long long bad;
-  auto load_chunk = [&]() {
-    const int j = (chunk << 6) + lane;
-    int pid = j < k.npg ? indices[k.pb + j] : 0;
-    asm volatile("" : "+v"(pid));  // the compiler's wait for this load stays here
+  auto page_id = [&](int c) {
+    const int j = (c << 6) + lane;
+    return j < k.npg ? indices[k.pb + j] : 0;
+  };
+  auto set_chunk = [&](int c, int pid) {
+    chunk = c;
     const bool out_of_pool = pid < 0 || pid >= num_pages;
     bad = __builtin_amdgcn_ballot_w64(out_of_pool);
     const uint64_t a = (uint64_t)(uintptr_t)(head0 + (int64_t)(out_of_pool ? 0 : pid) * 2 * plane_stride);
     pg_lo = (uint32_t)a;
     pg_hi = (uint32_t)(a >> 32);
   };
-  load_chunk();
+  const int chunk_beg = (t_beg / tpp) >> 6;  // of this workgroup's first tile (0 unless split > 0)
+  int pid0 = page_id(0), pid_beg = page_id(chunk_beg);
+  asm volatile("" : "+v"(pid0), "+v"(pid_beg));  // the compiler's wait for these loads stays here
+  set_chunk(0, pid0);
 #pragma unroll
   for (int s = 0; s < C::KS; ++s) asm volatile("" : "+v"(qb[s]));
 
@@ -1359,7 +1364,7 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
   // either: its tile is loaded from page 0 and, marked by -kTile tokens, cleared in LDS before use (weight 0 times any
   // byte of the pool could be NaN). Everything here is wave-uniform. Nearly every pair is two whole tiles of one page
   // and takes the short path (the general one on every pair: 188 us instead of 179 at 4096 tokens, HQ 16, HKV 2).
-  int cur_ti = t_beg, cur_lp = t_beg / tpp, cur_tp = t_beg - cur_lp * tpp;
+  int cur_ti = 0, cur_lp = 0, cur_tp = 0;
   const int t_whole = min(t_end, k.kv_len / kTile);  // tiles before this one are whole
   const int64_t tile_stride = kTile * row_stride;
   auto page_base = [&]() -> const unsigned char* {
@@ -1368,8 +1373,9 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
   };
   auto take = [&](int& nvalid) -> const unsigned char* {
     if ((cur_lp >> 6) != chunk) {  // the next 64 pages
-      chunk = cur_lp >> 6;
-      load_chunk();
+      int pid = page_id(cur_lp >> 6);
+      asm volatile("" : "+v"(pid));
+      set_chunk(cur_lp >> 6, pid);
     }
     const bool is_bad = (bad >> (cur_lp & 63)) & 1;
     const int got = min(kTile, (cur_lp == k.npg - 1 ? k.last : page_size) - cur_tp * kTile);
@@ -1477,9 +1483,25 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
     constexpr int AHEAD = kPfRing - 1;  // pairs in flight
     int na[AHEAD], nb[AHEAD];           // the valid tokens of their tiles
     auto rows_of = [&](int n) { return n > 0 ? n : 1; };
+    const unsigned char *ba, *bb;
+    // A later split takes its first softmax reference from the sequence's first pair, as the unsplit form does: the
+    // probabilities are then rounded to bf16 against the same reference, and the two forms agree to fp32 rounding
+    // (against its own first pair: 3e-3 of the output apart; with it 4e-5). The K rows of that pair land in the ring
+    // slot that is free until the first advance().
+    int ref_a = kTile, ref_b = kTile;
+    if (split > 0) {
+      take_pair(ba, bb, ref_a, ref_b);
+      if (plane == 0) {
+        tile_loads(ba, rows_of(ref_a), lds0 + AHEAD * C::PAIR);
+        tile_loads(bb, rows_of(ref_b), lds0 + AHEAD * C::PAIR + C::BUF);
+      }
+      cur_ti = t_beg;
+      cur_lp = t_beg / tpp;
+      cur_tp = t_beg - cur_lp * tpp;
+      set_chunk(chunk_beg, pid_beg);
+    }
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) {
-      const unsigned char *ba, *bb;
       take_pair(ba, bb, na[j], nb[j]);
       tile_loads(ba, rows_of(na[j]), lds0 + j * C::PAIR);
       tile_loads(bb, rows_of(nb[j]), lds0 + j * C::PAIR + C::BUF);
@@ -1494,8 +1516,9 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
       __builtin_amdgcn_s_barrier();
     };
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kPfRing - 2) * 2 * C::IPW) : "memory");
-    __builtin_amdgcn_s_barrier();  // every wave's loads of the first pair have landed
+    __builtin_amdgcn_s_barrier();  // every wave's loads of the first pair (and the reference pair) have landed
     clear_bad(na[0], nb[0], 0);
+    clear_bad(ref_a, ref_b, AHEAD);
     int slot = 0, slot_n;  // of pairs p and p + 1
     uint32_t dst;          // the slot of pair p - 1, which takes pair p + AHEAD
     const unsigned char *base_a, *base_b;
@@ -1522,15 +1545,17 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
       return;
     }
     float s[16];
-    {
+    auto first_scores = [&](int sl, int p, int a, int b) {  // the scores of pair p in ring slot sl, and their reference
       axk_f32x16 sn = zero16;
 #pragma unroll
-      for (int ks = 0; ks < C::KS; ++ks) sn = mfma_bf16_32x32x16(qk_frag(smem, ks), qb[ks], sn);
+      for (int ks = 0; ks < C::KS; ++ks) sn = mfma_bf16_32x32x16(qk_frag(smem + sl * C::PAIR, ks), qb[ks], sn);
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] = sn[i];
-      if (na[0] != kTile || nb[0] != kTile || 32 * p_beg + 31 > pos_lo) mask(s, p_beg, na[0], nb[0]);
+      if (a != kTile || b != kTile || 32 * p + 31 > pos_lo) mask(s, p, a, b);
       raise_max(row_max(s));
-    }
+    };
+    if (split > 0) first_scores(AHEAD, 0, ref_a, ref_b);
+    first_scores(0, p_beg, na[0], nb[0]);
     for (int p = p_beg; p < p_end; ++p) {
       advance();
       {

@@ -61,6 +61,23 @@ def test_split_matches_oracle_and_unsplit(dev, qlens, kv_lens, hq, hkv, d, page,
     assert torch.equal(got.view(torch.int16), _call(c, dev, True, scale).view(torch.int16))  # deterministic
 
 
+@pytest.mark.parametrize("qlens,kv_lens,hq,hkv,d,page", [
+    ([64], [4096], 16, 2, 256, 64),
+    ([4, 3, 2], [4096, 511, 900], 32, 4, 256, 64),
+    ([33, 1], [3000, 300], 8, 2, 128, 16),  # pairs crossing pages; pieces past the first 64 pages of a table
+    ([17], [9000], 16, 1, 64, 16),
+])
+def test_split_rounds_as_unsplit(dev, qlens, kv_lens, hq, hkv, d, page):
+    """A split's probabilities are rounded to bf16 against the sequence's own reference maximum, as the unsplit form's are,
+    so the two differ by fp32 sums alone: fewer than 1 % of the outputs round to the neighbouring bf16 value, and the
+    difference is below sqrt(0.01) 2^-8 of the output."""
+    g = torch.Generator().manual_seed(sum(kv_lens) + d)
+    c = configs.prefill_case(qlens, kv_lens, hq, hkv, d, page, g, extra_pages=2)
+    print(f"case qlens={qlens} kv_lens={kv_lens} hq={hq} hkv={hkv} d={d} page={page}", flush=True)
+    split, whole = (_call(c, dev, form, c["scale"]).double() for form in (True, False))
+    assert float((split - whole).norm() / whole.norm()) <= 0.1 * 2 ** -8
+
+
 def test_split_zero_scale_is_the_mean(dev):
     g = torch.Generator().manual_seed(8)
     c = configs.prefill_case([2], [900], 8, 2, 128, 64, g)
