@@ -1361,8 +1361,8 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
   }
   // the tile cursor: take_pair() gives the tiles two by two, in order (tile cur_tp of page cur_lp): their base
   // addresses and valid tokens; past t_end the last tile again with no tokens. A page outside the pool holds no tokens
-  // either: its tile is loaded from page 0 and, marked by -kTile tokens, cleared in LDS before use (weight 0 times any
-  // byte of the pool could be NaN). Everything here is wave-uniform. Nearly every pair is two whole tiles of one page
+  // either: its tile (also as the last tile again) is loaded from page 0 and, marked by -kTile tokens, cleared in LDS
+  // before use (weight 0 times any byte of the pool could be NaN). Everything here is wave-uniform. Nearly every pair is two whole tiles of one page
   // and takes the short path (the general one on every pair: 188 us instead of 179 at 4096 tokens, HQ 16, HKV 2).
   int cur_ti = 0, cur_lp = 0, cur_tp = 0;
   const int t_whole = min(t_end, k.kv_len / kTile);  // tiles before this one are whole
@@ -1380,7 +1380,7 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
     const bool is_bad = (bad >> (cur_lp & 63)) & 1;
     const int got = min(kTile, (cur_lp == k.npg - 1 ? k.last : page_size) - cur_tp * kTile);
     if (is_bad && status && lane == 0 && got > 0) *status = 1;
-    nvalid = cur_ti < t_end ? (is_bad ? -kTile : got) : 0;
+    nvalid = is_bad ? -kTile : cur_ti < t_end ? got : 0;
     const unsigned char* base = page_base();
     const int more = cur_ti + 1 < t_end, wrap = more && cur_tp + 1 == tpp;
     cur_tp = wrap ? 0 : cur_tp + more;

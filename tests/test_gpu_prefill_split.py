@@ -114,6 +114,34 @@ def test_bad_pages_hold_no_tokens(dev, split):
     assert int(status.item()) == 1
 
 
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("d,pages,last", [(128, 75, 16), (256, 21, 5)])
+def test_bad_last_page_of_an_odd_count(dev, d, pages, last, split):
+    """The last tile of an odd count is paired with itself: where its page is outside the pool and page 0 of the pool (whose
+    bytes it is loaded from) holds NaN, neither of the two reaches the output."""
+    g = torch.Generator().manual_seed(12)
+    page, t, hq, hkv = 16, 3, 8, 2
+    kv = (pages - 1) * page + last
+    c = configs.prefill_case([t], [kv], hq, hkv, d, page, g, extra_pages=1)
+    spare = [p for p in range(c["cache"].shape[0]) if p not in set(c["indices"].tolist())][0]
+    idx = c["indices"].clone()
+    idx[idx == 0] = spare
+    c["cache"][spare] = c["cache"][0]
+    c["cache"][0] = float("nan")
+    idx[-1] = c["cache"].shape[0]
+    c["indices"] = idx
+    # the new tokens lie on the last page (all of them with last >= t): each sees every token of the other pages
+    keys, values = (c["cache"][idx[:-1].long(), i].reshape(-1, hkv, d).float() for i in (0, 1))
+    rep = hq // hkv
+    s = torch.einsum("thd,khd->thk", c["q"].float(), keys.repeat_interleave(rep, 1)) * c["scale"]
+    ref = torch.einsum("thk,khd->thd", torch.softmax(s, -1), values.repeat_interleave(rep, 1))
+    status = torch.zeros(1, dtype=torch.int32, device=dev)
+    print(f"case bad last page d={d} pages={pages} split={split}", flush=True)
+    got = _call(c, dev, split, c["scale"], status)
+    torch.testing.assert_close(got.float(), ref.to(torch.bfloat16).float(), **TOL)
+    assert int(status.item()) == 1
+
+
 def test_layer_takes_a_workspace_without_the_splits(dev):
     """The verify layer runs in the buffers it cannot do without (the attention then unsplit), as with the full size."""
     g = torch.Generator().manual_seed(10)
