@@ -52,6 +52,7 @@ struct GdnArgs {
   float* snap;                  // optional: the state after token t at snap + t * snap_ld, [B, NV, DK, DV] each
   int64_t snap_ld;
   int kdiv;                     // value head h reads key head (h / kdiv) % NK
+  int out_over_qk;              // out overlaps q or k
 };
 
 // One token's inputs as a wave loads them: two rows of k and q a lane, v of the lane's columns, the gate inputs.
@@ -190,6 +191,7 @@ __global__ __launch_bounds__(kThreads, GATE && MULTI ? 3 : 4) void gdn_columns_k
     ov.z = row_group_sum(ov.z); ov.w = row_group_sum(ov.w);
     const float o = rg == 0 ? ov.x : rg == 1 ? ov.y : rg == 2 ? ov.z : ov.w;
     if (!GATE) {
+      if (p.out_over_qk) __syncthreads();  // every wave has this token's q and k before they are written over
       if (rg < 4) (p.out + vh)[col] = (uint16_t)f32_to_bf16_bits(o);
     } else {
       const float core = round_bf16(o);  // the head's bf16 output
@@ -380,6 +382,12 @@ int axk_gdn_recurrent_strided(const uint16_t* q, const uint16_t* k, const uint16
             (int)num_v_heads, ld.q, ld.k, ld.v, ld.ab, gate ? gate->norm_w : nullptr, gate ? gate->z : nullptr,
             gate ? gate->eps : 0.f, state_snap, snap_ld,
             v_order == AXK_VORDER_TILED ? 1 : (int)(num_v_heads / num_k_heads)};
+  // out may take the place of q, k or v (with as many key heads as value heads): a head's workgroup reads its token's
+  // rows before it writes them
+  auto over = [&](const uint16_t* x, int64_t row) {
+    return axk_overlap(out, obytes, x, (size_t)((batch * tokens - 1) * row + num_k_heads * kDK) * 2);
+  };
+  p.out_over_qk = over(q, ld.q) || over(k, ld.k);
   AXK_LAUNCH_GATE();
   // Which kernel, measured (32 value heads; us, rows in a loop over the tokens -> gdn_columns_kernel):
   //   1 token:  1 sequence 5.27 -> 4.65, 4 6.24 -> 5.37, 8 8.4 -> 7.5, 16 12.9 -> 11.8

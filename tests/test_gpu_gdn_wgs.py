@@ -5,7 +5,7 @@ import torch
 
 import test_gpu_gdn
 import test_gpu_layer
-from axk import configs, layer
+from axk import configs, gdn, layer
 from oracle import gdn as ogdn
 from oracle import layer as olayer
 
@@ -24,6 +24,19 @@ def test_gdn_workgroup_counts(dev, bsz, t, nk, nv, inplace):
     o32, s32 = ogdn.gdn_fp32(*test_gpu_gdn._args(c))
     torch.testing.assert_close(out.float(), o32.to(torch.bfloat16).float(), **test_gpu_gdn.TOL)
     torch.testing.assert_close(st, s32, rtol=1e-3, atol=1e-4)
+
+
+@pytest.mark.parametrize("over", ["q", "k", "v"])
+@pytest.mark.parametrize("bsz,t", [(3, 1), (3, 5), (20, 1), (40, 1)])
+def test_gdn_output_over_an_input(dev, bsz, t, over):
+    """As many key heads as value heads: the output in the place of q, k or v is the output in a tensor of its own, bit
+    for bit (each kernel of one token, and several tokens)."""
+    g = torch.Generator().manual_seed(bsz + t)
+    c = {n: x.to(dev) for n, x in configs.gdn_inputs(bsz, t, g, nk=16, nv=16, state_std=0.05).items()}
+    print(f"gdn output over {over} b={bsz} t={t}", flush=True)
+    want, state = gdn.gdn_recurrent(*test_gpu_gdn._args(c))
+    got, st = gdn.gdn_recurrent(*test_gpu_gdn._args(c), output=c[over])
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.equal(st, state)
 
 
 # With the output norm and gate: 256, 272, 512 and 544 workgroups. The layer rounds to bf16 some ten times between x and
