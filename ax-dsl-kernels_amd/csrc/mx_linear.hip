@@ -717,20 +717,42 @@ inline int64_t dg_blocks(const MxGroup& g, int epi) {
 
 // Where the dense GEMM is faster than the group kernel below 128 rows. The group kernel streams the weights once per 32
 // rows in many short workgroups, each reading its rows' whole activation; the GEMM once per call, in column blocks of
-// 256 whose K steps are a latency chain (0.5 us a step), so it needs enough of them. Measured (group kernel -> GEMM,
-// us; N x K, rows):
-//   MXFP4  24576 x 4096: 32 rows 41.3 -> 34.7;  16384 x 4096: 32 rows 28.1 -> 33.6, 64 rows 54.5 -> 33.7;
-//          8192 x 2048: 64 rows 19.4 -> 16.4, 100 rows 31.1 -> 17.2;  248320 x 2048: 32 rows 239 -> 87
-//   NVFP4  24576 x 4096: 32 rows 43.8 -> 41.9;  16384 x 4096: 64 rows 57.7 -> 41.9;  8192 x 2048: 64 rows 19.9 -> 24.2,
-//          100 rows 32.4 -> 24.5
-//   MXFP8  32768 x 4096: 32 rows 52.4 -> 63.0;  248320 x 2048: 32 rows 216 -> 117;  8192 x 2048: 64 rows 20.8 -> 18.5,
-//          100 rows 32.5 -> 18.5
+// 256 whose K steps are a latency chain (0.5 us a step), so it needs enough of them: more where the group kernel makes
+// a single pass, where weights decode slower (NVFP4) or are larger (8 bit), and where K is deep (the chain then costs
+// relatively more). Measured, group kernel's time over the GEMM's (17 / 32 rows; 33 / 48 / 64 rows; 65 rows; by blocks):
+//   MXFP4  K 2048:  64 blocks 0.77 / 0.90, 80 1.07 / 1.26;  32 blocks 0.90 / 1.02 / 1.19, 40 1.08 / 1.25 / 1.45;  32 1.35
+//          K 4096:  96 blocks 0.89 / 1.07, 128 1.11 / 1.32; 32 blocks 0.83 / 0.94 / 1.15, 48 0.91 / 1.08 / 1.18,
+//                   64 1.09 / 1.24 / 1.44;  32 1.34
+//          K 12288: 128 blocks 0.93 / 1.12, 160 1.09 / 1.29; 48 blocks 0.70 / 0.85 / 0.94, 64 0.92 / 1.05 / 1.22,
+//                   80 1.10 / 1.30 / 1.48;  32 1.27
+//   NVFP4  K 4096:  96 blocks 0.86 / 1.00, 128 1.10 / 1.29; 48 blocks 0.81 / 0.91 / 1.02, 64 1.00 / 1.11 / 1.33;  32 1.05
+//          K 12288: 128 blocks 0.91 / 1.05, 160 1.12 / 1.28; 64 blocks 0.82 / 0.94 / 1.10, 80 1.02 / 1.18 / 1.37;  32 1.07
+//   MXFP8  K 4096:  128 blocks 0.84 / 1.00, 192 1.07 / 1.28; 48 blocks 0.81 / 0.92 / 0.93, 64 0.97 / 1.02 / 1.15,
+//                   80 1.17 / 1.32 / 1.44;  32 1.05
+//          K 12288: 192 blocks 0.92 / 1.09, 256 1.12 / 1.37; 64 blocks 0.84 / 0.95 / 1.07, 80 1.02 / 1.17 / 1.28;  32 1.06
+//   FP8    K 4096:  128 blocks 0.92 / 1.09, 192 1.12 / 1.34; 33 blocks 0.89 / 1.02 / 1.25, 48 0.93 / 1.04 / 1.05,
+//                   64 1.15 / 1.23 / 1.32;  32 1.23
+//          K 12288: 192 blocks 0.88 / 1.19, 256 1.05 / 1.44; 48 blocks 0.75 / 0.90 / 0.91, 64 0.97 / 1.07 / 1.17,
+//                   80 1.11 / 1.28 / 1.37;  32 1.23
 template <int F>
-bool dg_rows(int64_t m, int64_t blocks) {
+bool dg_rows(int64_t m, int64_t blocks, int64_t k) {
+  constexpr bool mxfp4 = F == axk::WF_MXFP4, mx8 = axk::is_mx(F) && !mxfp4;
+  const bool deep = k > 4096;
   if (m >= kDgMinRows) return true;
   if (m <= 16) return false;
-  if (m <= 32) return blocks >= (axk::is_fp4(F) ? 96 : 192);
-  return blocks >= (axk::is_nv(F) && m <= 64 ? 64 : 32);
+  if (m <= 32) {
+    if (!axk::is_fp4(F)) return blocks >= (deep ? 256 : 192);
+    if (deep) return blocks >= 160;
+    const bool short_k = k <= 2048, full = m >= 28;  // (nearly a full pass of the group kernel)
+    return blocks >= ((mxfp4 ? short_k || full : short_k && full) ? 80 : 128);
+  }
+  if (m <= 64) {
+    if (mxfp4 && !deep) return blocks >= (m >= 56 ? 32 : m >= 48 ? 33 : m >= 40 ? 40 : 64);
+    if (F == axk::WF_FP8 && !deep) return blocks >= (m >= 48 ? 33 : 64);
+    if (deep) return blocks >= ((mxfp4 || F == axk::WF_FP8) && m >= 48 ? 64 : 80);
+    return blocks >= (mx8 && m < 40 ? 80 : 64);
+  }
+  return blocks >= 32;
 }
 
 // The dense GEMM for a checked group: one launch for all of its matrices (their column blocks end to end; EPI_SWIGLU
@@ -742,7 +764,7 @@ bool dg_fits(int64_t m, int64_t k, const AxkConvEpi* conv, const MxGroup& g, int
   if constexpr (F == axk::WF_BF16) {
     return false;
   } else {
-    if (conv != nullptr || k % kDgBK != 0 || !dg_rows<F>(m, dg_blocks(g, epi))) return false;
+    if (conv != nullptr || k % kDgBK != 0 || !dg_rows<F>(m, dg_blocks(g, epi), k)) return false;
     if constexpr (axk::is_mx(F)) {
       if (k % 128 != 0) return false;
       for (int i = 0; i < g.count; ++i)
