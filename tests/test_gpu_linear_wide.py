@@ -54,6 +54,25 @@ def test_rows_of_wide_matrices(dev, fmt, m, n, k):
     _close(got, a.float() @ wt.T + bias, out_dtype, a, wt)
 
 
+# What the group kernel, which sums K in eight runs, is off the exact product by, and a tenth: 6.1e-8 of the norm, 8.0e-8
+# where scale2 rounds once more, 1.21e-7 for codes of one sign.
+RUN_ERROR = {"mxfp4": 6.7e-8, "nvfp4": 8.8e-8, "e4m3": 1.33e-7}
+
+
+@pytest.mark.parametrize("fmt,m", [("mxfp4", 24), ("mxfp4", 100), ("nvfp4", 100)])
+def test_fp32_rows_are_summed_in_runs(dev, fmt, m):
+    """fp32 logits of an LM head's depth (K 2048) over 65536 channels are as near the exact product as the group kernel's,
+    whatever tile the rows take (one chain over K: 8.1e-8, 1.25e-7 with scale2)."""
+    a, got, bias, w = _run(fmt, m, 65536, 2048, torch.float32, dev)
+    x, err, norm = a.double(), 0.0, 0.0
+    for i in range(0, 65536, 8192):
+        ref = x @ torch.from_numpy(w[i:i + 8192]).double().T + bias[i:i + 8192].double()
+        err += float((got[:, i:i + 8192].cpu().double() - ref).square().sum())
+        norm += float(ref.square().sum())
+    print(f"{fmt} m={m} error {(err / norm) ** 0.5:.3g}", flush=True)
+    assert (err / norm) ** 0.5 <= RUN_ERROR[fmt]
+
+
 @pytest.mark.parametrize("mlp_fmt", ["mxfp4", "mxfp8"])
 def test_layer_mlp_of_40_rows(dev, mlp_fmt):
     """40 sequences, MLP width 4096: gate | up take the dense GEMM's SwiGLU form, the other projections the group's."""
