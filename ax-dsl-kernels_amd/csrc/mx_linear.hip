@@ -463,7 +463,8 @@ AXK_DEV void dg_decode(const unsigned char* row, int g4, int r, float sc, axk_bf
   }
 }
 
-template <int F, int EPI, int BM>
+// RUNS: fp32 outputs, summed in runs of K steps.
+template <int F, int EPI, int BM, bool RUNS>
 __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int RB = dg_row_bytes<F>(), STAGE = dg_stage<F, BM>();
@@ -586,8 +587,7 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
   static_assert(ST == 3, "the K loop is unrolled over three ring slots (every LDS offset an immediate)");
   // fp32 outputs of few rows are summed in eight runs of steps, the runs' sums apart, as the group kernel's eight waves
   // sum them: one chain over K is further from the exact sum (248320 x 2048, 32 rows: 7.8e-8 of it against 5.6e-8)
-  constexpr bool kRuns = EPI == EPI_PLAIN && BM <= 64;
-  axk_f32x4 tot[kRuns ? kDgMT : 1][4];
+  axk_f32x4 tot[RUNS ? kDgMT : 1][4];
   auto end_run = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int mt = 0; mt < kDgMT; ++mt)
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
         acc[mt][j] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
       }
   };
-  if constexpr (kRuns)
+  if constexpr (RUNS)
 #pragma unroll
     for (int mt = 0; mt < kDgMT; ++mt)
 #pragma unroll
@@ -607,13 +607,13 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
     step(ks, 0);
     if (ks + 1 < nk) step(ks + 1, 1);
     if (ks + 2 < nk) step(ks + 2, 2);
-    if constexpr (kRuns)
-      if (g.out_f32 && --left == 0) {
+    if constexpr (RUNS)
+      if (--left == 0) {
         end_run();
         left = run;
       }
   }
-  if constexpr (kRuns) {
+  if constexpr (RUNS) {
 #pragma unroll
     for (int mt = 0; mt < kDgMT; ++mt)
 #pragma unroll
@@ -778,15 +778,15 @@ bool dg_fits(int64_t m, int64_t k, const AxkConvEpi* conv, const MxGroup& g, int
   }
 }
 
-template <int F, int EPI, int BM>
+template <int F, int EPI, int BM, bool RUNS>
 int dg_launch(const DgArgs& d, int64_t nb, hipStream_t st) {
   static AxkOnce lds_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
-  if (const int rc = axk_raise_lds(lds_once, reinterpret_cast<const void*>(&mx_gemm_kernel<F, EPI, BM>), 160 * 1024))
+  if (const int rc = axk_raise_lds(lds_once, reinterpret_cast<const void*>(&mx_gemm_kernel<F, EPI, BM, RUNS>), 160 * 1024))
     return rc;
   const int64_t tiles = nb * (((int64_t)d.m + BM - 1) / BM);
   const int64_t grid = (tiles + kDgXcds - 1) / kDgXcds * kDgXcds;  // whole rounds over the XCDs
   AXK_REQUIRE(grid <= INT32_MAX, AXK_E_SHAPE);
-  hipLaunchKernelGGL((mx_gemm_kernel<F, EPI, BM>), dim3((unsigned)grid), dim3(256), (dg_lds_bytes<F, BM>()), st, d);
+  hipLaunchKernelGGL((mx_gemm_kernel<F, EPI, BM, RUNS>), dim3((unsigned)grid), dim3(256), (dg_lds_bytes<F, BM>()), st, d);
   return axk_launch_status();
 }
 
@@ -799,14 +799,14 @@ int dg_epi(const DgArgs& d, hipStream_t st) {
   constexpr int COLS = EPI == EPI_SWIGLU ? kDgBN / 2 : kDgBN;
   const int64_t nb = EPI == EPI_PLAIN ? d.cb0[d.count] : ((int64_t)d.n[0] + COLS - 1) / COLS;
   auto fills = [&](int bm) { return d.m > bm / 2 && nb * ((d.m + bm - 1) / bm) >= kDgCus; };
-  // fp32 outputs below kDgMinRows rows keep the run sums, which 128 rows' accumulators leave no registers for
-  // (100 rows of 248320 x 2048 MXFP4: 152 us at 128 rows and 8.1e-8 off the exact product, 179 us and 6.1e-8 at 64; the
-  // group kernel 815 us and 6.1e-8)
-  const bool runs = d.out_f32 && d.m < kDgMinRows;
+  // fp32 outputs are summed in runs in the tiles of 32 and 64 rows (128 rows' accumulators leave no registers for it), and
+  // below kDgMinRows rows they take no others (100 rows of 248320 x 2048 MXFP4: 152 us at 128 rows and 8.1e-8 off the
+  // exact product, 179 us and 6.1e-8 at 64; the group kernel 815 us and 6.1e-8)
   if constexpr (dg_bm<F>() > 64)
-    if (!runs && fills(dg_bm<F>())) return dg_launch<F, EPI, dg_bm<F>()>(d, nb, st);
-  if (fills(64)) return dg_launch<F, EPI, 64>(d, nb, st);
-  return dg_launch<F, EPI, 32>(d, nb, st);
+    if (!(d.out_f32 && d.m < kDgMinRows) && fills(dg_bm<F>())) return dg_launch<F, EPI, dg_bm<F>(), false>(d, nb, st);
+  if constexpr (EPI == EPI_PLAIN)
+    if (d.out_f32) return fills(64) ? dg_launch<F, EPI, 64, true>(d, nb, st) : dg_launch<F, EPI, 32, true>(d, nb, st);
+  return fills(64) ? dg_launch<F, EPI, 64, false>(d, nb, st) : dg_launch<F, EPI, 32, false>(d, nb, st);
 }
 
 template <int F>
