@@ -585,8 +585,9 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
     }
   };
   static_assert(ST == 3, "the K loop is unrolled over three ring slots (every LDS offset an immediate)");
-  // fp32 outputs of few rows are summed in eight runs of steps, the runs' sums apart, as the group kernel's eight waves
-  // sum them: one chain over K is further from the exact sum (248320 x 2048, 32 rows: 7.8e-8 of it against 5.6e-8)
+  // fp32 outputs of few rows are summed in eight runs of steps (a few more where K is no multiple of 512), the runs' sums
+  // apart, as the group kernel's eight waves sum them: one chain over K is further from the exact sum (248320 x 2048, 32
+  // rows: 7.8e-8 of it against 5.6e-8)
   axk_f32x4 tot[RUNS ? kDgMT : 1][4];
   auto end_run = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -602,16 +603,20 @@ __global__ __launch_bounds__(256, 2) void mx_gemm_kernel(DgArgs g) {
     for (int mt = 0; mt < kDgMT; ++mt)
 #pragma unroll
       for (int j = 0; j < 4; ++j) tot[mt][j] = axk_f32x4{0.f, 0.f, 0.f, 0.f};
-  const int run = (nk / 3 + 7) / 8;
-  for (int ks = 0, left = run; ks < nk; ks += 3) {
-    step(ks, 0);
-    if (ks + 1 < nk) step(ks + 1, 1);
-    if (ks + 2 < nk) step(ks + 2, 2);
+  const int run = max(1, nk / 8);
+  int left = run;
+  auto end_step = [&]() __attribute__((always_inline)) {
     if constexpr (RUNS)
       if (--left == 0) {
         end_run();
         left = run;
       }
+  };
+  for (int ks = 0; ks < nk; ks += 3) {
+    step(ks, 0);
+    end_step();
+    if (ks + 1 < nk) step(ks + 1, 1), end_step();
+    if (ks + 2 < nk) step(ks + 2, 2), end_step();
   }
   if constexpr (RUNS) {
 #pragma unroll
