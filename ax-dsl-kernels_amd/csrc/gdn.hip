@@ -31,7 +31,8 @@ constexpr int kLdRow = kRows + 4;        // floats between row groups of k / q i
 
 constexpr int kStepCols = kDV / 4;                  // gdn_recurrent_kernel: 32 threads across DV, 4 columns each
 constexpr int kStepRowGroups = kThreads / kStepCols;  // 8 row groups of kRows rows
-constexpr int kColsMaxWgs = 512, kEarlyMaxWgs = 256;  // see axk_gdn_recurrent_strided
+constexpr int kColsMaxWgs = 512, kEarlyMaxWgs = 256, kStepFullWgs = 2560;  // see axk_gdn_recurrent_strided
+constexpr int kStepPadLds = 54 * 1024;  // dynamic LDS that leaves room for two workgroups a CU
 
 struct GdnArgs {
   const uint16_t* q;   // [B, T, NK, DK] bf16
@@ -226,9 +227,11 @@ __global__ __launch_bounds__(kThreads, GATE && MULTI ? 3 : 4) void gdn_columns_k
 
 // One token for many sequences: the state's read and write fill the chip, and what counts is the order in which HBM
 // sees them. A wave reads and writes whole rows (two of 512 bytes an instruction), a workgroup's stores follow all of
-// its loads. Thread = 16 rows x 4 columns; the column sums meet in LDS.
+// its loads and start together. Thread = 16 rows x 4 columns; the column sums meet in LDS. (32 / 64 / 256 sequences of 32
+// heads: 24.1 / 47.2 / 190.7 us; without the barrier before the stores 24.2 / 48.4 / 195.9, with the compiler aiming at four
+// workgroups a CU 23.9 / 47.8 / 192.2.)
 template <bool GATE>
-__global__ __launch_bounds__(kThreads) void gdn_recurrent_kernel(GdnArgs p) {
+__global__ __launch_bounds__(kThreads, 3) void gdn_recurrent_kernel(GdnArgs p) {
   __shared__ float s_k[kDK], s_q[kDK];
   __shared__ float s_gn[2];
   __shared__ __align__(16) float s_red[kStepRowGroups / 2][kDV];  // per-wave partial column sums
@@ -342,6 +345,7 @@ __global__ __launch_bounds__(kThreads) void gdn_recurrent_kernel(GdnArgs p) {
     }
   }
 
+  __syncthreads();  // the workgroup's stores start together
   float* sout = p.state_out + ((int64_t)b * p.NV + h) * kDK * kDV;
 #pragma unroll
   for (int r = 0; r < kRows; ++r)
@@ -392,13 +396,15 @@ int axk_gdn_recurrent_strided(const uint16_t* q, const uint16_t* k, const uint16
   // Which kernel, measured (32 value heads; us, rows in a loop over the tokens -> gdn_columns_kernel):
   //   1 token:  1 sequence 5.27 -> 4.65, 4 6.24 -> 5.37, 8 8.4 -> 7.5, 16 12.9 -> 11.8
   //   4 tokens: 1 sequence 10.5 -> 9.7, 8 14.3 -> 13.4, 32 34.4 -> 32;  64 x 2 tokens of 16 heads 28.3 -> 27.8
-  // Above 512 workgroups of one token the state's traffic is all there is, and whole rows are the better order for it
-  // (32 sequences: 24.3 .. 25.6 us by rows, 26.9 by columns; 64: 50.2, by columns 50.5 with the inputs loaded first and
-  // 52.2 with the state first; rows in a loop over the tokens took 25.3 .. 26.5 and 49.5). From 257 workgroups, more
-  // than one a CU, the state is loaded first (16 sequences: 11.8 us,
-  // inputs first 13.8); up to 256 the inputs, whose chain is then the longer one.
+  // From 257 workgroups, more than one a CU, the state is loaded first (16 sequences: 11.8 us, inputs first 13.8); up to
+  // 256 the inputs, whose chain is then the longer one. Above 512 workgroups of one token the state's traffic is all there
+  // is, and whole rows are the better order for it (32 sequences: 24.1 us, 24.8 by columns; 64: 47.2, 49.1; rows in a loop
+  // over the tokens took 25.3 and 47.8, and 35.9 at 48 sequences, where this takes 36.4). Above 2560, where every CU has
+  // several rounds of them, two at a time are better than three: fewer reads and writes mix in HBM (96 sequences 70.0 ->
+  // 69.2 us, 128 92.9 -> 90.9, 256 190.7 -> 180.8; 80 58.7 -> 58.8, 64 47.2 -> 48.1).
   const dim3 grid((unsigned)(batch * num_v_heads));
-  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, p); };
+  auto launch = [&](auto kernel, int lds = 0) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), lds, stream, p); };
+  const int pad = grid.x > kStepFullWgs ? kStepPadLds : 0;
   if (tokens > 1 || state_snap)
     gate ? launch(gdn_columns_kernel<true, true, true>) : launch(gdn_columns_kernel<false, true, true>);
   else if (grid.x <= kEarlyMaxWgs)
@@ -406,7 +412,7 @@ int axk_gdn_recurrent_strided(const uint16_t* q, const uint16_t* k, const uint16
   else if (grid.x <= kColsMaxWgs)
     gate ? launch(gdn_columns_kernel<true, false, false>) : launch(gdn_columns_kernel<false, false, false>);
   else
-    gate ? launch(gdn_recurrent_kernel<true>) : launch(gdn_recurrent_kernel<false>);
+    gate ? launch(gdn_recurrent_kernel<true>, pad) : launch(gdn_recurrent_kernel<false>, pad);
   return axk_launch_status();
 }
 

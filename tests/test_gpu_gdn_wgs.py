@@ -1,4 +1,4 @@
-"""GPU parity of the GDN recurrent step on both sides of its kernel choice: 256 and 512 workgroups (sequences x value
+"""GPU parity of the GDN recurrent step on both sides of its kernel choice: 256, 512 and 2560 workgroups (sequences x value
 heads) of one token, and several tokens, which take the column kernel at every size. Tolerances as test_gpu_gdn.py."""
 import pytest
 import torch
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("inplace", [False, True])
 @pytest.mark.parametrize("bsz,t,nk,nv", [(16, 1, 16, 16), (257, 1, 1, 1), (32, 1, 8, 16), (27, 1, 1, 19),
-                                         (18, 2, 16, 32)])
+                                         (18, 2, 16, 32), (80, 1, 16, 32), (2561, 1, 1, 1)])
 def test_gdn_workgroup_counts(dev, bsz, t, nk, nv, inplace):
     g = torch.Generator().manual_seed(bsz + t)
     c = configs.gdn_inputs(bsz, t, g, nk=nk, nv=nv, state_std=0.05)
