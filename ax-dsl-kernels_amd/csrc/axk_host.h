@@ -99,10 +99,6 @@ __attribute__((visibility("hidden"))) int axk_conv_snapshots(const uint16_t* x, 
                                                              int64_t tokens, int64_t channels, int64_t kernel,
                                                              hipStream_t stream);
 
-// Internal (not exported): out[i] = i * step for i = 0 .. n (n + 1 values), int32 (a uniform row index, e.g. the
-// qo_indptr of `step` query rows per sequence). Returns an AXK status.
-__attribute__((visibility("hidden"))) int axk_fill_iota_i32(int32_t* out, int64_t n, int64_t step, hipStream_t stream);
-
 // Internal (not exported): one launch of up to AXK_MX_GROUP_MAX weight matrices that share the activations a
 // [m, k] (the projections of one decode layer). Matrix i: weights w [n, k] (FP8 bytes with a per-channel scale, or
 // MXFP4 codes / MXFP8 E4M3 bytes with E8M0 scales ws [n, k/32]), optional per-channel scale and bias, output
@@ -156,15 +152,15 @@ __attribute__((visibility("hidden"))) int axk_paged_decode_gated(
     int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages, float sm_scale, void* workspace,
     size_t workspace_bytes, hipStream_t stream);
 
-// Internal (not exported): axk_paged_prefill with the attention output gate applied where each output row is
-// written, as axk_paged_decode_gated (gate rows ldg elements apart, one per (token, query head) row). workspace (or
-// NULL): scratch of axk_paged_prefill_workspace_size bytes for the KV splits; with less the call does not split.
-// Returns an AXK status.
+// Internal (not exported): axk_paged_prefill of `tokens` new tokens in every sequence (rows b tokens + t of q) with the
+// attention output gate applied where each output row is written, as axk_paged_decode_gated (gate rows ldg elements apart,
+// one per (token, query head) row, 16-byte aligned, ldg a multiple of 8). workspace (or NULL): scratch of
+// axk_paged_prefill_workspace_size bytes for the KV splits; with less the call does not split. Returns an AXK status.
 __attribute__((visibility("hidden"))) int axk_paged_prefill_gated(
-    const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr, const int32_t* indptr,
-    const int32_t* indices, const int32_t* last_page_len, const uint16_t* gate, int64_t ldg, uint16_t* out,
-    int64_t batch, int64_t total_q, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
-    int64_t num_pages, float sm_scale, void* workspace, size_t workspace_bytes, hipStream_t stream);
+    const uint16_t* q, const uint16_t* kv_cache, const int32_t* indptr, const int32_t* indices,
+    const int32_t* last_page_len, const uint16_t* gate, int64_t ldg, uint16_t* out, int64_t batch, int64_t tokens,
+    int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages, float sm_scale,
+    void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 // Internal (not exported): axk_moe_decode with the shared expert computed by the caller: y_sh [tokens, hidden] fp32
 // is its down projection (any weight format), gated by sigmoid(h2 . w_shg) in the combine as the library's own

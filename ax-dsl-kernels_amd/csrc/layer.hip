@@ -436,12 +436,10 @@ GdnVerifyBufs carve_gdn_verify(Carver& c, int64_t R, int64_t H, int64_t NK, int6
 
 struct AttnVerifyBufs {
   uint16_t *h, *qg, *kk, *vv, *q, *attn, *gated, *y;
-  int32_t* qo_indptr;
   MlpBufs mlp;
 };
 
-AttnVerifyBufs carve_attn_verify(Carver& c, int64_t B, int64_t R, int64_t H, int64_t HQ, int64_t HKV, int64_t D,
-                                 int64_t F) {
+AttnVerifyBufs carve_attn_verify(Carver& c, int64_t R, int64_t H, int64_t HQ, int64_t HKV, int64_t D, int64_t F) {
   AttnVerifyBufs a;
   a.h = c.take<uint16_t>(R * H);
   a.qg = c.take<uint16_t>(R * HQ * 2 * D);
@@ -451,7 +449,6 @@ AttnVerifyBufs carve_attn_verify(Carver& c, int64_t B, int64_t R, int64_t H, int
   a.attn = c.take<uint16_t>(R * HQ * D);
   a.gated = c.take<uint16_t>(R * HQ * D);
   a.y = c.take<uint16_t>(R * H);
-  a.qo_indptr = c.take<int32_t>(B + 1);
   a.mlp = carve_mlp(c, R, H, F);
   return a;
 }
@@ -476,7 +473,7 @@ size_t attn_rows_ws(int64_t B, int64_t T, int64_t H, int64_t HQ, int64_t HKV, in
   if (HQ <= 0 || HKV <= 0 || HQ % HKV != 0 || !(D == 64 || D == 128 || D == 256)) return 0;
   if (moe && moe_ws_bytes(B * T, H, *moe) == 0) return 0;
   Carver c{nullptr};
-  carve_attn_verify(c, B, B * T, H, HQ, HKV, D, F);
+  carve_attn_verify(c, B * T, H, HQ, HKV, D, F);
   if (moe) carve_moe(c, B * T, H, *moe);
   if (splits) c.take<unsigned char>(axk_paged_prefill_workspace_size(B, B * T, HQ, HKV, D));
   return c.off;
@@ -505,7 +502,7 @@ int attn_rows_impl(const uint16_t* x, const float* ln1, const uint8_t* w_q, cons
   const int64_t B = batch, T = tokens, R = B * T, H = hidden, HQ = num_qo_heads, HKV = num_kv_heads, D = head_dim,
                 F = inter;
   Carver c{static_cast<unsigned char*>(workspace)};
-  const AttnVerifyBufs a = carve_attn_verify(c, B, R, H, HQ, HKV, D, F);
+  const AttnVerifyBufs a = carve_attn_verify(c, R, H, HQ, HKV, D, F);
   const MoeBufs eb = moe ? carve_moe(c, R, H, *moe) : MoeBufs{};
   unsigned char* split_ws = workspace_bytes > c.off ? c.base + c.off : nullptr;
   const size_t split_bytes = split_ws ? workspace_bytes - c.off : 0;
@@ -517,10 +514,9 @@ int attn_rows_impl(const uint16_t* x, const float* ln1, const uint8_t* w_q, cons
     AXK_TRY(projs(proj_fmt, a.h, H, proj, 3, R, H, stream));
     AXK_TRY(axk_attn_qkv_prep(a.qg, a.kk, a.vv, q_norm, k_norm, cos, sin, a.q, kv_cache, cache_location, R, HQ, HKV,
                               D, rot, page_size, num_pages, eps, axk_stream(stream)));
-    AXK_TRY(axk_fill_iota_i32(a.qo_indptr, B, T, axk_stream(stream)));
     // the attention with its output gate applied as each row is written: gated = bf16(attn * sigmoid(gate))
-    AXK_TRY(axk_paged_prefill_gated(a.q, kv_cache, a.qo_indptr, indptr, indices, last_page_len, a.qg + D, 2 * D,
-                                    a.gated, B, R, HQ, HKV, D, page_size, num_pages, sm_scale, split_ws, split_bytes,
+    AXK_TRY(axk_paged_prefill_gated(a.q, kv_cache, indptr, indices, last_page_len, a.qg + D, 2 * D, a.gated, B, T, HQ,
+                                    HKV, D, page_size, num_pages, sm_scale, split_ws, split_bytes,
                                     axk_stream(stream)));
     const AxkMxMat o = proj_mat(proj_fmt, w_o, s_o, a.y, H);
     AXK_TRY(projs(proj_fmt, a.gated, HQ * D, &o, 1, R, HQ * D, stream));

@@ -483,11 +483,6 @@ __global__ __launch_bounds__(256) void conv_snapshots_kernel(const uint16_t* __r
         *reinterpret_cast<const uint4*>(from + 8 * cc);
   }
 }
-
-__global__ __launch_bounds__(256) void fill_iota_kernel(int32_t* out, int n, int step) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i <= n) out[i] = i * step;
-}
 }  // namespace
 
 int axk_conv_snapshots(const uint16_t* x, const uint16_t* state_in, uint16_t* snap, int64_t snap_ld, int64_t batch,
@@ -502,14 +497,6 @@ int axk_conv_snapshots(const uint16_t* x, const uint16_t* state_in, uint16_t* sn
   AXK_LAUNCH_GATE();
   hipLaunchKernelGGL(conv_snapshots_kernel, dim3((unsigned)grid), dim3(256), 0, stream, x, state_in, snap, snap_ld,
                      (int)batch, (int)tokens, (int)channels, (int)kernel);
-  return axk_launch_status();
-}
-
-int axk_fill_iota_i32(int32_t* out, int64_t n, int64_t step, hipStream_t stream) {
-  AXK_REQUIRE(out, AXK_E_NULL);
-  AXK_REQUIRE(n >= 0 && n < INT32_MAX && step >= 0 && n * step <= INT32_MAX, AXK_E_SHAPE);
-  AXK_LAUNCH_GATE();
-  hipLaunchKernelGGL(fill_iota_kernel, dim3((unsigned)(n / 256 + 1)), dim3(256), 0, stream, out, (int)n, (int)step);
   return axk_launch_status();
 }
 

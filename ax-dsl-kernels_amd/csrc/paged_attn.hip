@@ -1142,9 +1142,10 @@ __global__ __launch_bounds__(256) void paged_kv_write_fp8_kernel(const uint16_t*
 // in that order.
 //
 // What bounds it: one wave issues at most one instruction every four cycles, and a pair's 32 MFMAs (1024 cycles)
-// bring about 300 others. Measured at D = 256, HQ 16, HKV 2: a 4096-token chunk 178 us, 773 TFLOP/s (237 us with 16
-// rows a wave, 16x16x32 MFMA and two waves a SIMD); 256 tokens after 16000 cached ones 98 us with the KV splits
-// (814 us before: 32 row blocks on 256 CUs).
+// bring about 300 others. Measured at D = 256, HQ 16, HKV 2: a 4096-token chunk 174 us, 790 TFLOP/s (237 us with 16
+// rows a wave, 16x16x32 MFMA and two waves a SIMD); 256 tokens after 16000 cached ones 96.5 us with the KV splits
+// (816 us before: 32 row blocks on 256 CUs). Short calls are bound by their chain: 1.4 us to the block's numbers, 0.9 to
+// the page ids, 2 to the first K / V, 1.1 a pair and 1.5 for the rows' way out (4 x 4 tokens of 64 cached ones 10.7 us).
 typedef short axk_s16x8 __attribute__((ext_vector_type(8)));
 typedef float axk_f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kPfWaves = 4;
@@ -1189,7 +1190,8 @@ AXK_DEV void for_each_index(F& f) {
 }
 
 // Row block `want` of one KV head: the blocks of each sequence in turn, its last (longest) block first. Every wave
-// derives the same answer; the grid is an upper bound and surplus workgroups get b = -1.
+// derives the same answer; the grid is an upper bound and surplus workgroups get b = -1. Without qo_indptr every sequence
+// has `tokens` new tokens. All of a sequence's numbers come in one round of loads, and the answer is wave-uniform.
 struct PfBlock {
   int b, r_first, r_last, q0, qlen;
   int pb, npg, last, kv_len;    // page range, valid tokens of the last page, cached tokens
@@ -1198,40 +1200,55 @@ struct PfBlock {
   int piece, ns;                // pairs per split of the sequence, splits this block has
 };
 
-AXK_DEV PfBlock pf_block(int want, const int* __restrict__ qo_indptr, const int* __restrict__ indptr,
+AXK_DEV PfBlock pf_block(int want, const int* __restrict__ qo_indptr, int tokens, const int* __restrict__ indptr,
                          const int* __restrict__ last_page_len, int batch, int group, int page_size, int nsplit) {
-  const int lane = threadIdx.x & 63;
   PfBlock k;
   k.b = -1;
-  int blk = 0;
-  for (int c0 = 0, base = 0; c0 < batch && k.b < 0; c0 += 64) {
-    const int sq = c0 + lane;
-    const int qlen_l = sq < batch ? qo_indptr[sq + 1] - qo_indptr[sq] : 0;
-    const int nb = qlen_l > 0 ? (qlen_l * group + kPfRows - 1) / kPfRows : 0;
-    int incl = nb;
+  int blk = 0, p_end = 0, last = 0;
+  if (qo_indptr == nullptr) {
+    const int nb = (tokens * group + kPfRows - 1) / kPfRows, b = want / nb;
+    if (b >= batch) return k;
+    k.b = b;
+    blk = nb - 1 - (want - b * nb);
+    k.q0 = b * tokens;
+    k.qlen = tokens;
+    k.pb = __builtin_amdgcn_readfirstlane(indptr[b]);
+    p_end = __builtin_amdgcn_readfirstlane(indptr[b + 1]);
+    last = __builtin_amdgcn_readfirstlane(last_page_len[b]);
+  } else {
+    const int lane = threadIdx.x & 63;
+    for (int c0 = 0, base = 0; c0 < batch && k.b < 0; c0 += 64) {
+      const int sq = c0 + lane, at = min(sq, batch - 1);
+      const int q_lo = qo_indptr[at], q_hi = qo_indptr[at + 1], p_lo = indptr[at], p_hi = indptr[at + 1];
+      const int last_l = last_page_len[at];
+      const int qlen_l = sq < batch ? q_hi - q_lo : 0;
+      const int nb = qlen_l > 0 ? (qlen_l * group + kPfRows - 1) / kPfRows : 0;
+      int incl = nb;
+      if (batch > 1)
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
+        for (int o = 1; o < 64; o <<= 1) {
+          const int v = __shfl_up(incl, o, 64);
+          if (lane >= o) incl += v;
+        }
+      const int excl = base + incl - nb;
+      const unsigned long long hit = __builtin_amdgcn_ballot_w64(nb > 0 && want >= excl && want < excl + nb);
+      if (hit) {
+        const int hl = __builtin_amdgcn_readfirstlane(__builtin_ctzll(hit));
+        auto of = [&](int v) { return __builtin_amdgcn_readlane(v, hl); };
+        k.b = c0 + hl;
+        blk = of(nb) - 1 - (want - of(excl));
+        k.q0 = of(q_lo);
+        k.qlen = of(qlen_l);
+        k.pb = of(p_lo);
+        p_end = of(p_hi);
+        last = of(last_l);
+      }
+      base += __builtin_amdgcn_readlane(incl, 63);
     }
-    const int excl = base + incl - nb;
-    const unsigned long long hit = __builtin_amdgcn_ballot_w64(nb > 0 && want >= excl && want < excl + nb);
-    if (hit) {
-      const int hl = __builtin_ctzll(hit);
-      k.b = c0 + hl;
-      blk = __shfl(nb, hl, 64) - 1 - (want - __shfl(excl, hl, 64));
-    }
-    base += __shfl(incl, 63, 64);
+    if (k.b < 0) return k;
   }
-  if (k.b < 0) return k;
-  k.b = __builtin_amdgcn_readfirstlane(k.b);
-  blk = __builtin_amdgcn_readfirstlane(blk);
-  // wave-uniform: scalar registers
-  k.q0 = __builtin_amdgcn_readfirstlane(qo_indptr[k.b]);
-  k.qlen = __builtin_amdgcn_readfirstlane(qo_indptr[k.b + 1]) - k.q0;
-  k.pb = __builtin_amdgcn_readfirstlane(indptr[k.b]);
-  k.npg = max(__builtin_amdgcn_readfirstlane(indptr[k.b + 1]) - k.pb, 0);
-  k.last = __builtin_amdgcn_readfirstlane(min(max(k.npg > 0 ? last_page_len[k.b] : 0, 0), page_size));
+  k.npg = max(p_end - k.pb, 0);
+  k.last = min(max(k.npg > 0 ? last : 0, 0), page_size);
   const int kv_len = k.kv_len = k.npg > 0 ? (k.npg - 1) * page_size + k.last : 0;
   const int tpp = page_size / kTile;
   k.r_first = blk * kPfRows;
@@ -1252,7 +1269,7 @@ AXK_DEV PfBlock pf_block(int want, const int* __restrict__ qo_indptr, const int*
 template <int D>
 __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefill_kernel(
     const uint16_t* __restrict__ q, const unsigned char* __restrict__ cache, const int* __restrict__ qo_indptr,
-    const int* __restrict__ indptr, const int* __restrict__ last_page_len, const int* __restrict__ indices,
+    int tokens, const int* __restrict__ indptr, const int* __restrict__ last_page_len, const int* __restrict__ indices,
     int batch, int total_q, int hq, int hkv, int page_size, int64_t num_pages, float sm_scale, int xcd_per_head,
     int nblk, int nsplit, int* __restrict__ status, uint16_t* __restrict__ out, const uint16_t* __restrict__ gate,
     int64_t ldg, float2* __restrict__ part_ml, float* __restrict__ part_o) {
@@ -1282,7 +1299,7 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, l32 = lane & 31, h = lane >> 5;
 
-  const PfBlock k = pf_block(want, qo_indptr, indptr, last_page_len, batch, group, page_size, nsplit);
+  const PfBlock k = pf_block(want, qo_indptr, tokens, indptr, last_page_len, batch, group, page_size, nsplit);
   if (k.b < 0 || split >= k.ns) return;
   if (k.q0 < 0 || k.q0 + k.qlen > total_q) {  // a query range outside q: nothing is read or written
     if (status && threadIdx.x == 0) *status = 1;
@@ -1506,7 +1523,10 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
       tile_loads(ba, rows_of(na[j]), lds0 + j * C::PAIR);
       tile_loads(bb, rows_of(nb[j]), lds0 + j * C::PAIR + C::BUF);
     }
-    const int p_beg = t_beg / 2, p_end = (t_end + 1) / 2;
+    // the loop below takes pairs p_beg .. p_last - 1; at D <= 128 the last pair has code of its own (4096 tokens, HQ 8, HKV 2,
+    // D 128: 122 -> 114 us, a single pair 7.7 -> 6.7; at D = 256 that costs the loop 7 % of its time: 176 -> 189 us)
+    constexpr bool kPeel = D <= 128;
+    const int p_beg = t_beg / 2, p_last = (t_end + 1) / 2 - (kPeel ? 1 : 0);
     // the pair with tokens (a, b) in ring slot sl has landed for every wave: clear its tiles of pages outside the pool
     auto clear_bad = [&](int a, int b, int sl) {
       if (a >= 0 && b >= 0) return;
@@ -1535,7 +1555,7 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
       ra = rows_of(na[AHEAD - 1]), rb = rows_of(nb[AHEAD - 1]);
     };
     if (!active) {  // no rows (the end of a row block): this wave only loads its share
-      for (int p = p_beg; p < p_end; ++p) {
+      for (int p = p_beg; p < p_last; ++p) {
         advance();
         tile_loads(base_a, ra, dst);
         tile_loads(base_b, rb, dst + C::BUF);
@@ -1556,27 +1576,35 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
     };
     if (split > 0) first_scores(AHEAD, 0, ref_a, ref_b);
     first_scores(0, p_beg, na[0], nb[0]);
-    for (int p = p_beg; p < p_end; ++p) {
+    // V^T tile j mod DT of the pair's 16-token tile j / DT (x: vx)
+    auto pv_frag = [&](const unsigned char* vb, int x, int j) {
+      const int t = j % C::DT;
+      const unsigned char* va = vb + vaddr + 64 * ((t & 3) ^ x) + 256 * (t >> 2) + (j / C::DT) * C::BUF;
+      const axk_s16x4 v0 = lds_read_tr16(va), v1 = lds_read_tr16(va + 8 * C::RB);
+      return __builtin_bit_cast(axk_bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    float m_use;  // a row that has seen nothing stays at zero: its scores are all -inf and exp2(-inf) = 0
+    auto prob = [&](int i) {
+      s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -m_use));
+      l_run += s[i];
+    };
+    auto pack_probs = [&](int ti) {
+      axk_u32x4 w;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(s[8 * ti + 2 * i], s[8 * ti + 2 * i + 1]);
+      return __builtin_bit_cast(axk_bf16x8, w);
+    };
+    for (int p = p_beg; p < p_last; ++p) {
       advance();
       {
         const unsigned char* kb = smem + slot_n * C::PAIR;
         const unsigned char* vb = smem + slot * C::PAIR;
-        auto pv_frag = [&](int j) {  // V^T tile j mod DT of the pair's 16-token tile j / DT
-          const int t = j % C::DT;
-          const unsigned char* va = vb + vaddr + 64 * ((t & 3) ^ vx) + 256 * (t >> 2) + (j / C::DT) * C::BUF;
-          const axk_s16x4 v0 = lds_read_tr16(va), v1 = lds_read_tr16(va + 8 * C::RB);
-          return __builtin_bit_cast(axk_bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-        };
-        // a row that has seen nothing stays at zero: its scores are all -inf and exp2(-inf) = 0
-        const float m_use = m_run == -INFINITY ? 0.f : m_run;
+        m_use = m_run == -INFINITY ? 0.f : m_run;
         axk_f32x16 sn = zero16;
         axk_bf16x8 kf[KA], vf[VA], pf[2];
         auto probs = [&](int lo, int hi) {
 #pragma unroll
-          for (int i = lo; i < hi; ++i) {
-            s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c, -m_use));
-            l_run += s[i];
-          }
+          for (int i = lo; i < hi; ++i) prob(i);
           asm volatile("" : "+v"(l_run));  // the sum stays in this stage
         };
 #pragma unroll
@@ -1588,7 +1616,7 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
           sn = mfma_bf16_32x32x16(kf[I % KA], qb[I], sn);
           asm volatile("" : "+a"(sn));  // this MFMA stays in this stage (and the accumulators in AGPRs)
           if constexpr (I + KA < C::KS) kf[I % KA] = qk_frag(kb, I + KA);
-          else if constexpr (I + KA - C::KS < VA) vf[I + KA - C::KS] = pv_frag(I + KA - C::KS);
+          else if constexpr (I + KA - C::KS < VA) vf[I + KA - C::KS] = pv_frag(vb, vx, I + KA - C::KS);
           if constexpr (I < C::IPW) tile_load(std::integral_constant<int, I % C::IPW>{}, base_a, ra, dst);
           else if constexpr (I < 2 * C::IPW)
             tile_load(std::integral_constant<int, I % C::IPW>{}, base_b, rb, dst + C::BUF);
@@ -1597,21 +1625,16 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
         };
         for_each_index<C::KS>(qk_stage);
 #pragma unroll
-        for (int i = KA; i < VA; ++i) vf[i] = pv_frag(i);
+        for (int i = KA; i < VA; ++i) vf[i] = pv_frag(vb, vx, i);
 #pragma unroll
-        for (int ti = 0; ti < 2; ++ti) {
-          axk_u32x4 w;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(s[8 * ti + 2 * i], s[8 * ti + 2 * i + 1]);
-          pf[ti] = __builtin_bit_cast(axk_bf16x8, w);
-        }
+        for (int ti = 0; ti < 2; ++ti) pf[ti] = pack_probs(ti);
         __builtin_amdgcn_sched_barrier(0);
         float mx = -INFINITY;
 #pragma unroll
         for (int j = 0; j < PV; ++j) {
           o[j % C::DT] = mfma_bf16_32x32x16(vf[j % VA], pf[j / C::DT], o[j % C::DT]);
           asm volatile("" : "+a"(o[j % C::DT]));
-          if (j + VA < PV) vf[j % VA] = pv_frag(j + VA);
+          if (j + VA < PV) vf[j % VA] = pv_frag(vb, vx, j + VA);
           if (j >= 2)
 #pragma unroll
             for (int i = 16 * (j - 2) / (PV - 2); i < 16 * (j - 1) / (PV - 2); ++i) {
@@ -1630,6 +1653,24 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
       }
       slot = slot_n;
     }
+    if constexpr (kPeel) {  // the last pair: nothing to load or score beside it
+      const unsigned char* vb = smem + slot * C::PAIR;
+      m_use = m_run == -INFINITY ? 0.f : m_run;
+      int x = vx;
+      asm volatile("" : "+v"(x));  // its addresses are formed here, and no register of the loop above holds them
+      axk_bf16x8 vf[VA];
+#pragma unroll
+      for (int i = 0; i < VA; ++i) vf[i] = pv_frag(vb, x, i);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) prob(i);
+      const axk_bf16x8 pf[2] = {pack_probs(0), pack_probs(1)};
+#pragma unroll
+      for (int j = 0; j < PV; ++j) {
+        o[j % C::DT] = mfma_bf16_32x32x16(vf[j % VA], pf[j / C::DT], o[j % C::DT]);
+        asm volatile("" : "+a"(o[j % C::DT]));  // (in AGPRs, as above)
+        if (j + VA < PV) vf[j % VA] = pv_frag(vb, x, j + VA);
+      }
+    }
     wait_vmcnt<0>();
   }
 
@@ -1647,32 +1688,54 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
             make_float4(o[t][4 * i], o[t][4 * i + 1], o[t][4 * i + 2], o[t][4 * i + 3]);
     return;
   }
+  // Lanes l and l + 32 exchange halves, so that each holds 8 columns of two: 32 t + 16 i + 8 h of its row, a 16-byte store
+  // (and gate load: 128 loads of 2 bytes a lane took 13 us of a verify layer's attention, one store a 4-column piece 3 us
+  // of every call).
   const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+  const bool out16 = ((uintptr_t)out & 15) == 0;  // else 8-byte aligned
+  uint16_t* const orow = out + qrow * D + 8 * h;
+  axk_u32x4 gw[2 * C::DT];
+  if (gate) {
 #pragma unroll
-  for (int t = 0; t < C::DT; ++t)
+    for (int i = 0; i < 2 * C::DT; ++i)
+      gw[i] = *reinterpret_cast<const axk_u32x4*>(gate + qrow * ldg + 16 * i + 8 * h);
+  }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int col = 32 * t + 8 * i + 4 * h;
-      const int64_t gi = qrow * ldg + col;  // (with a gate)
-      uint2 w;
-      w.x = gated_bf16(o[t][4 * i] * inv, gate, gi) | (gated_bf16(o[t][4 * i + 1] * inv, gate, gi + 1) << 16);
-      w.y = gated_bf16(o[t][4 * i + 2] * inv, gate, gi + 2) | (gated_bf16(o[t][4 * i + 3] * inv, gate, gi + 3) << 16);
-      *reinterpret_cast<uint2*>(out + qrow * D + col) = w;
+  for (int i = 0; i < 2 * C::DT; ++i) {
+    const auto& ot = o[i / 2];
+    const int e = 8 * (i % 2);
+    const auto w0 = __builtin_amdgcn_permlane32_swap(pack_bf16x2(ot[e] * inv, ot[e + 1] * inv),
+                                                     pack_bf16x2(ot[e + 4] * inv, ot[e + 5] * inv), false, false);
+    const auto w1 = __builtin_amdgcn_permlane32_swap(pack_bf16x2(ot[e + 2] * inv, ot[e + 3] * inv),
+                                                     pack_bf16x2(ot[e + 6] * inv, ot[e + 7] * inv), false, false);
+    axk_u32x4 w = {w0[0], w1[0], w0[1], w1[1]};
+    if (gate) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        w[j] = pack_bf16x2(bf16_bits_to_f32(w[j] & 0xffffu) * sigmoid_f32(bf16_bits_to_f32(gw[i][j] & 0xffffu)),
+                           bf16_bits_to_f32(w[j] >> 16) * sigmoid_f32(bf16_bits_to_f32(gw[i][j] >> 16)));
     }
+    if (out16) {
+      *reinterpret_cast<axk_u32x4*>(orow + 16 * i) = w;
+    } else {
+      *reinterpret_cast<uint2*>(orow + 16 * i) = make_uint2(w[0], w[1]);
+      *reinterpret_cast<uint2*>(orow + 16 * i + 4) = make_uint2(w[2], w[3]);
+    }
+  }
 }
 
 // The log-sum-exp merge of the splits of each row (as paged_merge_kernel): one wave per row, kPfMergeRows rows of one
 // row block per workgroup. Row blocks with a single split wrote their output already.
 template <int D>
 __global__ __launch_bounds__(256) void paged_prefill_merge_kernel(
-    const int* __restrict__ qo_indptr, const int* __restrict__ indptr, const int* __restrict__ last_page_len,
-    int batch, int total_q, int hq, int hkv, int page_size, int nsplit, const float2* __restrict__ part_ml,
+    const int* __restrict__ qo_indptr, int tokens, const int* __restrict__ indptr,
+    const int* __restrict__ last_page_len, int batch, int total_q, int hq, int hkv, int page_size, int nsplit, const float2* __restrict__ part_ml,
     const float* __restrict__ part_o, uint16_t* __restrict__ out, const uint16_t* __restrict__ gate, int64_t ldg) {
   constexpr int PER = D / 64;  // columns per lane
   const int group = hq / hkv;
   constexpr int SUB = kPfRows / kPfMergeRows;
   const int sub = blockIdx.x % SUB, kvh = blockIdx.x / SUB % hkv, want = blockIdx.x / SUB / hkv;
-  const PfBlock k = pf_block(want, qo_indptr, indptr, last_page_len, batch, group, page_size, nsplit);
+  const PfBlock k = pf_block(want, qo_indptr, tokens, indptr, last_page_len, batch, group, page_size, nsplit);
   if (k.b < 0 || k.ns <= 1 || k.q0 < 0 || k.q0 + k.qlen > total_q) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int i = wave; i < kPfMergeRows; i += 4) {
@@ -1729,14 +1792,15 @@ size_t pf_ws_bytes(int64_t batch, int64_t total_q, int64_t hq, int64_t hkv, int6
 }
 
 template <int D>
-int launch_prefill(const uint16_t* q, const void* cache, const int* qo_indptr, const int* indptr, const int* last,
-                   const int* indices, uint16_t* out, int batch, int total_q, int hq, int hkv, int page_size,
+int launch_prefill(const uint16_t* q, const void* cache, const int* qo_indptr, int tokens, const int* indptr,
+                   const int* last, const int* indices, uint16_t* out, int batch, int total_q, int hq, int hkv, int page_size,
                    int64_t num_pages, float sm_scale, int* status, hipStream_t st, const uint16_t* gate, int64_t ldg,
                    void* ws) {
   const int64_t rows = (int64_t)total_q * (hq / hkv);
   const int ns = ws ? pf_splits(batch, total_q, hq, hkv) : 1;
-  // >= the sum over sequences of their row blocks (one sequence: exactly)
-  const int64_t nblk = (rows + kPfRows - 1) / kPfRows + (batch > 1 ? batch : 0);
+  // >= the sum over sequences of their row blocks (one sequence, or as many rows in each: exactly)
+  const int64_t nblk = qo_indptr ? (rows + kPfRows - 1) / kPfRows + (batch > 1 ? batch : 0)
+                                 : batch * (((int64_t)tokens * (hq / hkv) + kPfRows - 1) / kPfRows);
   const int xph = hkv <= 8 && 8 % hkv == 0 ? 8 / hkv : 0;  // XCDs per KV head
   const int64_t grid = xph ? 8 * ((nblk * ns + xph - 1) / xph) : nblk * ns * hkv;
   if (grid > 0x7fffffff) return AXK_E_SHAPE;
@@ -1747,11 +1811,11 @@ int launch_prefill(const uint16_t* q, const void* cache, const int* qo_indptr, c
   float* po = reinterpret_cast<float*>(ml + (ws ? (int64_t)ns * total_q * hq : 0));
   AXK_LAUNCH_GATE();
   hipLaunchKernelGGL((paged_prefill_kernel<D>), dim3((unsigned)grid), dim3(64 * kPfWaves), lds, st, q,
-                     static_cast<const unsigned char*>(cache), qo_indptr, indptr, last, indices, batch, total_q, hq,
+                     static_cast<const unsigned char*>(cache), qo_indptr, tokens, indptr, last, indices, batch, total_q, hq,
                      hkv, page_size, num_pages, sm_scale, xph, (int)nblk, ns, status, out, gate, ldg, ml, po);
   if (ns > 1)
     hipLaunchKernelGGL((paged_prefill_merge_kernel<D>), dim3((unsigned)(nblk * hkv * (kPfRows / kPfMergeRows))),
-                       dim3(256), 0, st, qo_indptr, indptr, last, batch, total_q, hq, hkv, page_size, ns, ml, po, out,
+                       dim3(256), 0, st, qo_indptr, tokens, indptr, last, batch, total_q, hq, hkv, page_size, ns, ml, po, out,
                        gate, ldg);
   return axk_launch_status();
 }
@@ -2308,13 +2372,14 @@ extern "C" int axk_paged_kv_write_i8(const uint16_t* k, const uint16_t* v, int8_
 // themselves. flash_attn.py:471-611 (paged_flash_attention: history pages, then the causal current block),
 // q35_prefill.py:264-336 (the G x P-row block attention per KV head).
 namespace {
-// axk_paged_prefill, with the optional attention output gate applied as each row is written (gate rows ldg apart).
-int prefill_impl(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr, const int32_t* indptr,
-                 const int32_t* indices, const int32_t* last_page_len, uint16_t* out, int64_t batch, int64_t total_q,
+// axk_paged_prefill, with the optional attention output gate applied as each row is written (gate rows ldg apart);
+// tokens > 0: that many new tokens in every sequence, and no qo_indptr.
+int prefill_impl(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr, int64_t tokens,
+                 const int32_t* indptr, const int32_t* indices, const int32_t* last_page_len, uint16_t* out, int64_t batch, int64_t total_q,
                  int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages,
                  float sm_scale, int32_t* status, hipStream_t st, const uint16_t* gate, int64_t ldg, void* workspace,
                  size_t workspace_bytes) {
-  AXK_REQUIRE(q && kv_cache && qo_indptr && indptr && indices && last_page_len && out, AXK_E_NULL);
+  AXK_REQUIRE(q && kv_cache && (qo_indptr || tokens > 0) && indptr && indices && last_page_len && out, AXK_E_NULL);
   AXK_REQUIRE(batch > 0 && batch <= (1 << 20) && total_q >= 0 && total_q <= (1 << 24), AXK_E_SHAPE);
   AXK_REQUIRE(num_kv_heads > 0 && num_qo_heads > 0 && num_qo_heads % num_kv_heads == 0, AXK_E_SHAPE);
   AXK_REQUIRE(num_kv_heads <= 4096 && total_q * num_qo_heads <= ((int64_t)1 << 31) / 256, AXK_E_SHAPE);
@@ -2331,13 +2396,13 @@ int prefill_impl(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_
   const int B = (int)batch, T = (int)total_q, HQ = (int)num_qo_heads, HKV = (int)num_kv_heads, PS = (int)page_size;
   switch (head_dim) {
     case 64:
-      return launch_prefill<64>(q, kv_cache, qo_indptr, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
+      return launch_prefill<64>(q, kv_cache, qo_indptr, (int)tokens, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
                                 num_pages, sm_scale, status, st, gate, ldg, ws);
     case 128:
-      return launch_prefill<128>(q, kv_cache, qo_indptr, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
+      return launch_prefill<128>(q, kv_cache, qo_indptr, (int)tokens, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
                                  num_pages, sm_scale, status, st, gate, ldg, ws);
     default:
-      return launch_prefill<256>(q, kv_cache, qo_indptr, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
+      return launch_prefill<256>(q, kv_cache, qo_indptr, (int)tokens, indptr, last_page_len, indices, out, B, T, HQ, HKV, PS,
                                  num_pages, sm_scale, status, st, gate, ldg, ws);
   }
 }
@@ -2348,7 +2413,7 @@ extern "C" int axk_paged_prefill(const uint16_t* q, const uint16_t* kv_cache, co
                                  uint16_t* out, int64_t batch, int64_t total_q, int64_t num_qo_heads,
                                  int64_t num_kv_heads, int64_t head_dim, int64_t page_size, int64_t num_pages,
                                  float sm_scale, int32_t* status, axk_stream_t stream) {
-  return prefill_impl(q, kv_cache, qo_indptr, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
+  return prefill_impl(q, kv_cache, qo_indptr, 0, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
                       num_kv_heads, head_dim, page_size, num_pages, sm_scale, status, axk_stream(stream), nullptr, 0,
                       nullptr, 0);
 }
@@ -2371,24 +2436,23 @@ extern "C" int axk_paged_prefill_split(const uint16_t* q, const uint16_t* kv_cac
   AXK_REQUIRE(workspace_bytes >=
                   axk_paged_prefill_workspace_size(batch, total_q, num_qo_heads, num_kv_heads, head_dim),
               AXK_E_WORKSPACE);
-  return prefill_impl(q, kv_cache, qo_indptr, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
+  return prefill_impl(q, kv_cache, qo_indptr, 0, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
                       num_kv_heads, head_dim, page_size, num_pages, sm_scale, status, axk_stream(stream), nullptr, 0,
                       workspace, workspace_bytes);
 }
 
-int axk_paged_prefill_gated(const uint16_t* q, const uint16_t* kv_cache, const int32_t* qo_indptr,
-                            const int32_t* indptr, const int32_t* indices, const int32_t* last_page_len,
-                            const uint16_t* gate, int64_t ldg, uint16_t* out, int64_t batch, int64_t total_q,
-                            int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim, int64_t page_size,
-                            int64_t num_pages, float sm_scale, void* workspace, size_t workspace_bytes,
-                            hipStream_t stream) {
+int axk_paged_prefill_gated(const uint16_t* q, const uint16_t* kv_cache, const int32_t* indptr, const int32_t* indices,
+                            const int32_t* last_page_len, const uint16_t* gate, int64_t ldg, uint16_t* out,
+                            int64_t batch, int64_t tokens, int64_t num_qo_heads, int64_t num_kv_heads, int64_t head_dim,
+                            int64_t page_size, int64_t num_pages, float sm_scale, void* workspace,
+                            size_t workspace_bytes, hipStream_t stream) {
   AXK_REQUIRE(gate, AXK_E_NULL);
-  AXK_REQUIRE(ldg >= head_dim, AXK_E_SHAPE);
-  if (total_q > 0) {
-    const size_t gbytes = (size_t)((total_q * num_qo_heads - 1) * ldg + head_dim) * 2;
-    AXK_REQUIRE(!axk_overlap(out, (size_t)total_q * num_qo_heads * head_dim * 2, gate, gbytes), AXK_E_ALIAS);
-  }
-  return prefill_impl(q, kv_cache, qo_indptr, indptr, indices, last_page_len, out, batch, total_q, num_qo_heads,
-                      num_kv_heads, head_dim, page_size, num_pages, sm_scale, nullptr, stream, gate, ldg, workspace,
-                      workspace_bytes);
+  AXK_REQUIRE(batch > 0 && tokens > 0 && tokens <= (1 << 24) / batch && ldg >= head_dim, AXK_E_SHAPE);
+  AXK_REQUIRE(axk_aligned(gate, 16) && ldg % 8 == 0, AXK_E_ALIGN);
+  const int64_t rows = batch * tokens * num_qo_heads;
+  AXK_REQUIRE(!axk_overlap(out, (size_t)rows * head_dim * 2, gate, (size_t)((rows - 1) * ldg + head_dim) * 2),
+              AXK_E_ALIAS);
+  return prefill_impl(q, kv_cache, nullptr, tokens, indptr, indices, last_page_len, out, batch, batch * tokens,
+                      num_qo_heads, num_kv_heads, head_dim, page_size, num_pages, sm_scale, nullptr, stream, gate, ldg,
+                      workspace, workspace_bytes);
 }

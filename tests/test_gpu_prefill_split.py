@@ -78,6 +78,25 @@ def test_split_rounds_as_unsplit(dev, qlens, kv_lens, hq, hkv, d, page):
     assert float((split - whole).norm() / whole.norm()) <= 0.1 * 2 ** -8
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("kv", [30, 32, 33, 70])
+def test_output_8_byte_aligned(dev, d, kv):
+    """Contexts of one pair of tiles, of a whole pair and of a token more; an output that is 8-byte aligned only (its rows
+    then leave in 8-byte pieces) holds the same bits as an aligned one."""
+    g = torch.Generator().manual_seed(d + kv)
+    c = _dev(configs.prefill_case([5, 2], [kv, kv + 3], 8, 2, d, 16, g), dev)
+    args = (c["q"], c["cache"], c["qo_indptr"], c["indptr"], c["indices"], c["last_page_len"])
+    want = attention.paged_prefill(*args)
+    ref = pa.paged_prefill(*(t.cpu() for t in args), c["scale"])
+    torch.testing.assert_close(want.float().cpu(), ref.to(torch.bfloat16).float(), **TOL)
+    pool = torch.full((c["q"].numel() + 8,), float("nan"), dtype=torch.bfloat16, device=dev)
+    out = pool[4:4 + c["q"].numel()].view_as(c["q"])
+    assert out.data_ptr() % 16 == 8
+    attention.paged_prefill(*args, output=out)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert pool[:4].isnan().all() and pool[4 + c["q"].numel():].isnan().all()
+
+
 def test_split_zero_scale_is_the_mean(dev):
     g = torch.Generator().manual_seed(8)
     c = configs.prefill_case([2], [900], 8, 2, 128, 64, g)
