@@ -336,11 +336,13 @@ def paged_prefill(
             last_page_len.data_ptr(), output.data_ptr(), b, t, hq, hkv, d, page, p, float(sm_scale),
             _lib.ptr(status))
     # few row blocks over a long history: the cached tokens are split over more workgroups (fp32 partials in a scratch
-    # tensor). Up to 320 cached tokens (the page table bounds them) a split is one or two pieces of 256 and its merge
-    # launch costs more than it gives (32 new tokens, HQ 16, HKV 2, D 256: at 232 cached tokens 20.9 us unsplit, 23.5
-    # split).
+    # tensor), but the merge launch, and a workgroup for every split, cost more than they give where sequences are short
+    # (unsplit / split, us, at 320, 448 and 640 cached tokens each, HQ 16, HKV 2, D 256: 1 sequence of 32 new tokens 21.4 /
+    # 25.5, 25.8 / 25.5, 32.6 / 26.1; 16 of 4 19.5 / 23.4, 23.7 / 23.5, 30.1 / 24.1; 32 of 4 19.6 / 27.1, 24.1 / 27.1,
+    # 30.7 / 28.0). All that is known of the lengths here is their sum, from the page table's capacity; the line lies
+    # below the measured one since the longest of several sequences, which counts, is above their mean.
     scratch = 0
-    if indices.numel() * page > 320:
+    if indices.numel() * page > 384 + 320 * (b - 1):
         scratch = _lib.load().axk_paged_prefill_workspace_size(b, t, hq, hkv, d)
     if scratch:
         ws = torch.empty(scratch, dtype=torch.uint8, device=q.device)

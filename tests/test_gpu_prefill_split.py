@@ -203,3 +203,17 @@ def test_split_under_capture(dev):
         torch.cuda.synchronize()
         assert torch.equal(out.cpu().view(torch.int16), want.view(torch.int16))
         torch.randn(1 << 20, device=dev).sum().item()
+
+
+@pytest.mark.parametrize("qlens,kv_lens,split", [([4] * 8, [100] * 8, False), ([4], [320], False), ([4], [448], True),
+                                                 ([4] * 8, [320] * 7 + [448], True)])
+def test_short_sequences_are_not_split(dev, monkeypatch, qlens, kv_lens, split):
+    """The operator splits by the cached tokens a sequence has room for, not by their sum."""
+    c = _dev(configs.prefill_case(qlens, kv_lens, 16, 2, 128, 64, torch.Generator().manual_seed(3)), dev)
+    names, call = [], _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *args: (names.append(name), call(name, *args))[1])
+    got = attention.paged_prefill(c["q"], c["cache"], c["qo_indptr"], c["indptr"], c["indices"], c["last_page_len"])
+    assert names == ["axk_paged_prefill_split" if split else "axk_paged_prefill"]
+    ref = pa.paged_prefill(*(c[n].cpu() for n in ("q", "cache", "qo_indptr", "indptr", "indices", "last_page_len")),
+                           c["scale"])
+    torch.testing.assert_close(got.float().cpu(), ref.to(torch.bfloat16).float(), **TOL)
