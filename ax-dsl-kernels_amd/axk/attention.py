@@ -290,6 +290,13 @@ def store_paged_kv_i8(k: torch.Tensor, v: torch.Tensor, kv_cache: torch.Tensor, 
     )
 
 
+def paged_prefill_workspace(batch: int, total_q: int, num_qo_heads: int, num_kv_heads: int, head_dim: int,
+                            device) -> torch.Tensor:
+    """A byte buffer large enough for paged_prefill with this configuration (empty where it never splits)."""
+    n = _lib.load().axk_paged_prefill_workspace_size(batch, total_q, num_qo_heads, num_kv_heads, head_dim)
+    return torch.empty(n, dtype=torch.uint8, device=device)
+
+
 def paged_prefill(
     q: torch.Tensor,
     kv_cache: torch.Tensor,
@@ -300,12 +307,19 @@ def paged_prefill(
     sm_scale: Optional[float] = None,
     output: Optional[torch.Tensor] = None,
     status: Optional[torch.Tensor] = None,
+    workspace: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """Causal attention of several new tokens per sequence over the paged cache (prefill chunks, speculative verify):
     q bf16 [T, HQ, D] holds sequence b's new tokens in rows qo_indptr[b] .. qo_indptr[b + 1]; their K / V are already
     in the cache as the sequence's last tokens, so new token t of a sequence of kv_len cached tokens sees positions
     0 .. kv_len - qlen + t (flash_attn.py:471-611, q35_prefill.py:264-336). Returns bf16 [T, HQ, D]. A page id
-    outside the pool or a query range outside q sets status (device int32 [1], if given) to 1."""
+    outside the pool or a query range outside q sets status (device int32 [1], if given) to 1.
+
+    Few rows over a long history are split over the chip through scratch memory: workspace (a byte buffer of
+    paged_prefill_workspace, kept by the caller), or else a tensor allocated by the call; with a smaller workspace, or
+    without the memory for one, the call runs unsplit. Whether it splits follows from the shapes and the page table's
+    capacity (indices.numel() x page size), since the lengths are on the device: a table padded to its maximum counts as
+    full."""
     _check(q.dim() == 3 and q.dtype == torch.bfloat16 and q.is_contiguous(), "q must be contiguous bf16 [T, HQ, D]")
     _check(kv_cache.dim() == 5 and kv_cache.dtype == torch.bfloat16 and kv_cache.is_contiguous(),
            "kv_cache must be contiguous bf16 [pages, 2, page_size, HKV, D]")
@@ -331,6 +345,9 @@ def paged_prefill(
     if status is not None:
         _check(status.dtype == torch.int32 and status.numel() >= 1, "status must be int32 [1]")
         tensors.append(status)
+    if workspace is not None:
+        _check(workspace.dtype == torch.uint8 and workspace.is_contiguous(), "workspace must be contiguous uint8")
+        tensors.append(workspace)
     _lib.require_device(*tensors)
     args = (q.data_ptr(), kv_cache.data_ptr(), qo_indptr.data_ptr(), indptr.data_ptr(), indices.data_ptr(),
             last_page_len.data_ptr(), output.data_ptr(), b, t, hq, hkv, d, page, p, float(sm_scale),
@@ -341,12 +358,16 @@ def paged_prefill(
     # 25.5, 25.8 / 25.5, 32.6 / 26.1; 16 of 4 19.5 / 23.4, 23.7 / 23.5, 30.1 / 24.1; 32 of 4 19.6 / 27.1, 24.1 / 27.1,
     # 30.7 / 28.0). All that is known of the lengths here is their sum, from the page table's capacity; the line lies
     # below the measured one since the longest of several sequences, which counts, is above their mean.
-    scratch = 0
+    ws, scratch = workspace, 0
     if indices.numel() * page > 384 + 320 * (b - 1):
         scratch = _lib.load().axk_paged_prefill_workspace_size(b, t, hq, hkv, d)
-    if scratch:
-        ws = torch.empty(scratch, dtype=torch.uint8, device=q.device)
-        _lib.call("axk_paged_prefill_split", *args, ws.data_ptr(), scratch, _lib.stream_of(q))
+    if scratch and ws is None:
+        try:
+            ws = torch.empty(scratch, dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:
+            pass
+    if scratch and ws is not None and ws.numel() >= scratch:
+        _lib.call("axk_paged_prefill_split", *args, ws.data_ptr(), ws.numel(), _lib.stream_of(q))
     else:
         _lib.call("axk_paged_prefill", *args, _lib.stream_of(q))
     return output

@@ -217,3 +217,32 @@ def test_short_sequences_are_not_split(dev, monkeypatch, qlens, kv_lens, split):
     ref = pa.paged_prefill(*(c[n].cpu() for n in ("q", "cache", "qo_indptr", "indptr", "indices", "last_page_len")),
                            c["scale"])
     torch.testing.assert_close(got.float().cpu(), ref.to(torch.bfloat16).float(), **TOL)
+
+
+def test_workspace_of_the_caller(dev, monkeypatch):
+    """A kept workspace takes the place of the call's own scratch, bit for bit, and nothing is allocated; without the memory
+    for a scratch, or with a smaller workspace, the call runs unsplit."""
+    c = _dev(configs.prefill_case([4, 3], [900, 1500], 16, 2, 128, 64, torch.Generator().manual_seed(4)), dev)
+    args = (c["q"], c["cache"], c["qo_indptr"], c["indptr"], c["indices"], c["last_page_len"])
+    want = attention.paged_prefill(*args)
+    ws = attention.paged_prefill_workspace(2, 7, 16, 2, 128, dev)
+    assert ws.numel() > 0 and attention.paged_prefill_workspace(2, 4096, 16, 2, 128, dev).numel() == 0
+    out = torch.empty_like(want)
+    before = torch.cuda.memory_stats(dev)["allocation.all.allocated"]
+    attention.paged_prefill(*args, output=out, workspace=ws)
+    assert torch.cuda.memory_stats(dev)["allocation.all.allocated"] == before
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    whole = _call(c, dev, False, c["scale"]).to(dev)
+    attention.paged_prefill(*args, output=out, workspace=ws[:-1])
+    assert torch.equal(out.view(torch.int16), whole.view(torch.int16))
+
+    def no_memory(*args, **kw):
+        raise torch.OutOfMemoryError()
+
+    out.zero_()
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", no_memory)
+        attention.paged_prefill(*args, output=out)
+    assert torch.equal(out.view(torch.int16), whole.view(torch.int16))
+    with pytest.raises(ValueError):
+        attention.paged_prefill(*args, workspace=ws.view(torch.int32) if ws.numel() % 4 == 0 else ws[::2])
