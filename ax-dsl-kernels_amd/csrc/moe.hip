@@ -58,13 +58,14 @@ constexpr int kDecodeTokens = 64 * kMaskWords;  // above this the prefill path r
 constexpr int64_t kMaxPrefillTokens = 1 << 16;
 constexpr int64_t kMaxPrefillPairs = 1 << 19;
 constexpr int kBlkTokens = 256;  // tokens per block of the prefill grouping
-constexpr int kBM = 128, kBK = 64;  // prefill GEMM: most rows of a tile, K step
+constexpr int kBM = 128, kBK = 64;  // prefill GEMM: rows of a tile where experts have many, K step
 // The rows of a tile: 32 or 64 where the experts' rows are few on average (T K / E), so that the GEMMs neither load nor
 // multiply tiles that are mostly padding. Measured (E 256, top-8, H 2048, F 512; us with 32- / 64- / 128-row tiles):
 // 257 tokens 182 / 193 / 216, 700 tokens 196 / 206 / 227, 1024 tokens 227 / 216 / 236, 1400 tokens 266 / 227 / 246,
 // 2048 tokens 320 / 273 / 272, 4096 tokens 544 / 428 / 408. Around 128 rows an expert, half the experts have a few more
 // than a 128-row tile takes, and their second tiles stream and decode the weights again: 160-row tiles there (4096
-// tokens 426 -> 397 us on one box; 2800 tokens, whose experts fit 128 rows, 328 -> 348).
+// tokens 426 -> 397 us on one box; 2800 tokens, whose experts fit 128 rows, 328 -> 348). At the band's edges: 3850 tokens
+// (120.3 rows an expert) 379 us, 3840 in 128 rows 381; 5280 (165) 515, 5300 in 128 rows 518.
 constexpr int kBMWide = 160;
 inline int tile_rows(int64_t T, int64_t E, int64_t K) {
   const int64_t p = T * K;
@@ -135,8 +136,8 @@ MoeWs moe_ws(void* ws, int64_t T, int64_t H, int64_t E, int64_t K, int64_t F, in
   size_t off[kWsParts];
   moe_ws_layout(T, H, E, K, F, Fs, off);
   unsigned char* b = reinterpret_cast<unsigned char*>(ws);
-  // a list of 32- or 64-row tiles, longer than its part, takes the half of y that bf16 rows leave (T K H bytes a half,
-  // the list at most T K / 2 + 16 E + T / 2 + 48)
+  // a list of 32- or 64-row tiles, longer than its part, takes the half of y that bf16 rows leave (2 T K H bytes, H at
+  // least 64; the list at most T K / 2 + 16 E + T / 2 + 48, E at most 1024)
   const size_t tiles = T > kDecodeTokens && tile_rows(T, E, K) < kBM ? off[9] + (size_t)T * K * H * 2 : off[12];
   return {reinterpret_cast<int*>(b + off[0]),       reinterpret_cast<int*>(b + off[1]),
           reinterpret_cast<int4*>(b + off[2]),      reinterpret_cast<int*>(b + off[3]),
@@ -588,15 +589,13 @@ struct GateUpArgs {
 
 // gate-up + SwiGLU: workgroup (slot, ngrp-th run of kStreamWaves * tpw tiles); wave w streams tiles
 // run + w + kStreamWaves i.
-// WIDE (K a multiple of the batch's 128 kBatchChunks values): a batch's E8M0 scales are 4 kBatchChunks
-// consecutive bytes of the row (chunks x lane groups), fetched with one load per matrix; otherwise one byte load
-// per unit.
-// STAGE (with WIDE): each batch's weights are loaded as whole row segments of 64 kBatchChunks bytes (16 / kBatchChunks
-// rows per load instruction, which keeps the address path's per-line work low), written to a wave-private LDS tile
-// and read back in the MFMA layout; ROWS activation rows per pass.
-template <bool WIDE, int ROWS, bool STAGE>
+// STAGE (K a multiple of the batch's 128 kBatchChunks values): each batch's weights are loaded as whole row segments of
+// 64 kBatchChunks bytes (16 / kBatchChunks rows per load instruction, which keeps the address path's per-line work low),
+// written to a wave-private LDS tile and read back in the MFMA layout, and its E8M0 scales, 4 kBatchChunks consecutive
+// bytes of the row (chunks x lane groups), come with one load per matrix. Otherwise weights and scales are loaded unit by
+// unit. ROWS activation rows per pass.
+template <int ROWS, bool STAGE>
 __global__ __launch_bounds__(kStreamThreads) void moe_gateup_kernel(GateUpArgs a) {
-  static_assert(!STAGE || WIDE, "staged weights need whole batches");
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ SlotLds L;
   uint16_t* sA = reinterpret_cast<uint16_t*>(smem);
@@ -668,13 +667,11 @@ __global__ __launch_bounds__(kStreamThreads) void moe_gateup_kernel(GateUpArgs a
         const int64_t kb = min((int64_t)(bi * kBatchChunks + j) * 128 + 32 * g, (int64_t)H - 32);
         bt.qg[j] = load_nt(past ? idle + 32 * j : gw + n * (H / 2) + kb / 2);
         bt.qu[j] = load_nt(past ? idle + 32 * j + 16 : uw + n * (H / 2) + kb / 2);
-        if (!WIDE) {
-          bt.sg[j] = gs[n * (H / 32) + kb / 32];
-          bt.su[j] = us[n * (H / 32) + kb / 32];
-        }
+        bt.sg[j] = gs[n * (H / 32) + kb / 32];
+        bt.su[j] = us[n * (H / 32) + kb / 32];
       }
     }
-    if (WIDE) {
+    if (STAGE) {
       load_scale_words(bt.sg, gs + n * (H / 32) + 4 * kBatchChunks * bi);
       load_scale_words(bt.su, us + n * (H / 32) + 4 * kBatchChunks * bi);
     }
@@ -708,12 +705,12 @@ __global__ __launch_bounds__(kStreamThreads) void moe_gateup_kernel(GateUpArgs a
 #pragma unroll
       for (int j = 0; j < kBatchChunks; ++j) {
         const int c = bi * kBatchChunks + j;
-        if (!WIDE && c * 128 >= H) continue;  // whole chunk past K (uniform)
+        if (!STAGE && c * 128 >= H) continue;  // whole chunk past K (uniform)
         const int kb = c * 128 + 32 * g;
-        const bool kv = WIDE || kb < H;       // this lane's unit (a chunk can straddle the end of K)
+        const bool kv = STAGE || kb < H;       // this lane's unit (a chunk can straddle the end of K)
         const int kc = kv ? kb : H - 32;
-        const uint32_t bg = WIDE ? (cur.sg[j] >> (8 * g)) & 0xffu : cur.sg[j];
-        const uint32_t bu = WIDE ? (cur.su[j] >> (8 * g)) & 0xffu : cur.su[j];
+        const uint32_t bg = STAGE ? (cur.sg[j] >> (8 * g)) & 0xffu : cur.sg[j];
+        const uint32_t bu = STAGE ? (cur.su[j] >> (8 * g)) & 0xffu : cur.su[j];
         const float scg = kv ? e8m0_to_f32(bg) : 0.f, scu = kv ? e8m0_to_f32(bu) : 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -777,9 +774,8 @@ struct DownArgs {
 };
 
 // down: workgroup (slot, run of kStreamWaves * tpw 16-row tiles of H); routed rows scaled by their routing weight.
-template <bool WIDE, int ROWS, bool STAGE>
+template <int ROWS, bool STAGE>
 __global__ __launch_bounds__(kStreamThreads) void moe_down_kernel(DownArgs a) {
-  static_assert(!STAGE || WIDE, "staged weights need whole batches");
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ SlotLds L;
   uint16_t* sA = reinterpret_cast<uint16_t*>(smem);
@@ -843,10 +839,10 @@ __global__ __launch_bounds__(kStreamThreads) void moe_down_kernel(DownArgs a) {
       for (int j = 0; j < kBatchChunks; ++j) {
         const int64_t kb = min((int64_t)(bi * kBatchChunks + j) * 128 + 32 * g, (int64_t)K - 32);
         bt.q[j] = load_nt(past ? idle + 16 * j : dw + n * (K / 2) + kb / 2);
-        if (!WIDE) bt.s[j] = ds[n * (K / 32) + kb / 32];
+        bt.s[j] = ds[n * (K / 32) + kb / 32];
       }
     }
-    if (WIDE) load_scale_words(bt.s, ds + n * (K / 32) + 4 * kBatchChunks * bi);
+    if (STAGE) load_scale_words(bt.s, ds + n * (K / 32) + 4 * kBatchChunks * bi);
   };
 
   int m0 = mbeg;
@@ -891,11 +887,11 @@ __global__ __launch_bounds__(kStreamThreads) void moe_down_kernel(DownArgs a) {
 #pragma unroll
       for (int j = 0; j < kBatchChunks; ++j) {
         const int c = bi * kBatchChunks + j;
-        if (!WIDE && c * 128 >= K) continue;
+        if (!STAGE && c * 128 >= K) continue;
         const int kb = c * 128 + 32 * g;
-        const bool kv = WIDE || kb < K;
+        const bool kv = STAGE || kb < K;
         const int kc = kv ? kb : K - 32;
-        const uint32_t sb = WIDE ? (cur.s[j] >> (8 * g)) & 0xffu : cur.s[j];
+        const uint32_t sb = STAGE ? (cur.s[j] >> (8 * g)) & 0xffu : cur.s[j];
         const float sc = kv ? e8m0_to_f32(sb) : 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -1174,19 +1170,19 @@ __global__ __launch_bounds__(256) void moe_pscatter_kernel(const int32_t* __rest
 }
 
 // ---------------------------------------------------------------------------------------------
-// prefill grouped GEMM: workgroup (tile of kBM rows of one expert, 256 weight rows), wave w a 64 x 64 block of
-// the output (four 16-row x four 16-column MFMA tiles: every A fragment feeds four MFMAs and every B fragment
-// four). MODE 0: weight rows = 128 gate + the same 128 up columns (SwiGLU pairs gate and up tiles in the same
+// prefill grouped GEMM: workgroup (BM rows of a TB-row tile of one expert, 256 weight rows), wave w a BM x 64 block of
+// the output (BM / 16 16-row x four 16-column MFMA tiles: every A fragment feeds four MFMAs and every B fragment
+// BM / 16). MODE 0: weight rows = 128 gate + the same 128 up columns (SwiGLU pairs gate and up tiles in the same
 // lanes); MODE 1: 256 columns of H.
 // The A rows (gathered by token) and the packed weights of each 64-wide K step land in LDS by direct loads (no
-// register staging) into a ring of kGStages steps, two steps ahead, with one barrier per step; the E8M0 scales of
-// the whole reduction are staged once per workgroup. A stage holds A [64 rows][128 B] with the 16-byte chunk c of
-// row r at position c ^ (r & 7), and B [256 weight rows][32 B] with the 16-byte half h of row r at position
-// h ^ ((r >> 3) & 1): the fragment reads of either are then free of bank conflicts. Workgroups are mapped so that
-// all tiles and column blocks of one expert run on one XCD: its weights are fetched into that XCD's L2 once.
+// register staging) into a ring of kGStages steps, kGStages - 1 ahead, with one barrier per step. A stage holds A
+// [BM rows][128 B] with the 16-byte chunk c of row r at position c ^ (r & 7), and B [256 weight rows][32 B] with the
+// 16-byte half h of row r at position h ^ ((r >> 3) & 1): the fragment reads of either are then free of bank conflicts.
+// Workgroups are mapped so that all tiles and column blocks of one expert run on one XCD: its weights are fetched into
+// that XCD's L2 once.
 // SDMA (reductions of whole 128-element scale dwords, 4-byte aligned scales): each step's E8M0 bytes come with the
-// step's direct loads, one dword per weight row, LDS kGStages x (A 8 KiB + B 8 KiB + 1 KiB), so three workgroups
-// share a CU; otherwise the scales of the whole reduction are staged once, LDS kGStages x 16 KiB + [256][Kd/32 + 16].
+// step's direct loads, one dword per weight row, LDS kGStages x (A BM x 128 B + B 8 KiB + 1 KiB); otherwise the scales
+// of the whole reduction are staged once, LDS kGStages x (A + B) + [256][Kd / 32 + 16].
 // ---------------------------------------------------------------------------------------------
 struct GGemmArgs {
   const uint16_t* a;     // gate-up: h2 [T, H]; down: act [P, F]
@@ -1598,13 +1594,12 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   const int run_gu = kStreamWaves * gu_tpw, run_dn = kStreamWaves * dn_tpw;
   const int gu_grp = ((fmax + 15) / 16 + run_gu - 1) / run_gu;
   const int dn_grp = ((H + 15) / 16 + run_dn - 1) / run_dn;
-  const int wide_k = 128 * kBatchChunks;
-  const bool gu_wide = H % wide_k == 0, dn_wide = F % wide_k == 0 && Fs % wide_k == 0;
+  const int batch_k = 128 * kBatchChunks;
   const size_t stage_lds = kStreamWaves * kWaveStageBytes;
   const bool many = T > 64;  // (a size that 16 unstaged rows would not fit is refused there, staged or not)
   AXK_REQUIRE(!many || (stream_stage_off(kStageRows, H) <= kMaxStreamLds &&
                         stream_stage_off(kStageRows, fmax) <= kMaxStreamLds), AXK_E_SHAPE);
-  const bool gu_stage = gu_wide, dn_stage = dn_wide;
+  const bool gu_stage = H % batch_k == 0, dn_stage = F % batch_k == 0 && Fs % batch_k == 0;
   const bool gu_mid = gu_stage && many && (int64_t)T * K > 5 * (int64_t)E &&
                       stream_stage_off(kMidRows, H) + stage_lds <= kMaxStreamLds;
   const bool dn_full = dn_stage && many && (int64_t)T * K > 4 * (int64_t)E &&
@@ -1616,12 +1611,12 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   AXK_REQUIRE(gu_lds <= kMaxStreamLds && dn_lds <= kMaxStreamLds, AXK_E_SHAPE);
   static AxkOnce lds_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
   const int raised = axk_once(lds_once, [] {
-    const void* fns[6] = {reinterpret_cast<const void*>(&moe_gateup_kernel<true, kMidRows, true>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<true, kStageRows, true>),
-                          reinterpret_cast<const void*>(&moe_gateup_kernel<false, kStageRows, false>),
-                          reinterpret_cast<const void*>(&moe_gateup_kernel<true, kSmallRows, true>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<false, kStageRows, false>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<true, kSmallRows, true>)};
+    const void* fns[6] = {reinterpret_cast<const void*>(&moe_gateup_kernel<kMidRows, true>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<kStageRows, true>),
+                          reinterpret_cast<const void*>(&moe_gateup_kernel<kStageRows, false>),
+                          reinterpret_cast<const void*>(&moe_gateup_kernel<kSmallRows, true>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<kStageRows, false>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<kSmallRows, true>)};
     for (const void* f : fns) {
       const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxStreamLds);
       if (e != hipSuccess) return e;
@@ -1634,18 +1629,18 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
                 gu_nsp, w};
   const dim3 gu_grid((unsigned)((max_slots + gu_nsp) * gu_grp)), dn_grid((unsigned)((max_slots + dn_nsp) * dn_grp));
   if (gu_mid)
-    hipLaunchKernelGGL((moe_gateup_kernel<true, kMidRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+    hipLaunchKernelGGL((moe_gateup_kernel<kMidRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   else if (gu_stage)
-    hipLaunchKernelGGL((moe_gateup_kernel<true, kSmallRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+    hipLaunchKernelGGL((moe_gateup_kernel<kSmallRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   else
-    hipLaunchKernelGGL((moe_gateup_kernel<false, kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+    hipLaunchKernelGGL((moe_gateup_kernel<kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   DownArgs da{e_dw, e_ds, sh_down_w, sh_down_s, topk_ids, topk_weights, T, H, F, Fs, E, K, dn_grp, dn_tpw, dn_nsp, w};
   if (dn_full)
-    hipLaunchKernelGGL((moe_down_kernel<true, kStageRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+    hipLaunchKernelGGL((moe_down_kernel<kStageRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   else if (dn_stage)
-    hipLaunchKernelGGL((moe_down_kernel<true, kSmallRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+    hipLaunchKernelGGL((moe_down_kernel<kSmallRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   else
-    hipLaunchKernelGGL((moe_down_kernel<false, kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+    hipLaunchKernelGGL((moe_down_kernel<kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   // the decode router formed the shared gate's logit when the routing ran in this call (gate_given)
   CombineArgs ca{h2, x_res, w_shg, gate_given ? w.gate_logit : nullptr, topk_ids, combine_shared, T, H, E, K, w, out};
   launch_combine<false>(ca, st);
