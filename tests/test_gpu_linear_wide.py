@@ -1,6 +1,7 @@
 """GPU parity of the runtime-weight linears at 17 .. 127 rows of wide matrices, where the dense GEMM takes over from the
-group kernel: both sides of each threshold, every tile of rows (32, 64, 128) at its edges, ragged channel counts, and a
-decode layer whose MLP takes the SwiGLU form. Bars as tests/test_gpu_linear_prefill.py."""
+group kernel: both sides of each threshold with the tile of 32 rows, the tiles of 64 and 128 rows (which need 256 workgroups)
+at their edges in each epilogue, ragged channel counts, and a decode layer whose MLP takes the SwiGLU form. Bars as
+tests/test_gpu_linear_prefill.py."""
 import pytest
 import torch
 
@@ -54,9 +55,35 @@ def test_rows_of_wide_matrices(dev, fmt, m, n, k):
     _close(got, a.float() @ wt.T + bias, out_dtype, a, wt)
 
 
+# Workgroups are ceil(n / 256) x ceil(m / rows), and the tile is the largest that gives 256 of them: 64 rows at (40, ..) and
+# (1000, ..), 128 at the others in 4 bit (64 in 8 bit, which has no more).
+@pytest.mark.parametrize("fmt", ["mxfp4", "nvfp4", "fp8", "e4m3"])
+@pytest.mark.parametrize("m,n,k,out_dtype", [(40, 65550, 128, torch.bfloat16), (64, 65536, 128, torch.float32),
+                                             (70, 65550, 128, torch.bfloat16), (130, 33000, 256, torch.float32),
+                                             (1000, 4100, 256, torch.bfloat16), (2100, 4104, 256, torch.bfloat16)])
+def test_tiles_of_64_and_128_rows(dev, fmt, m, n, k, out_dtype):
+    print(f"{fmt} m={m} n={n} k={k} {out_dtype}", flush=True)
+    a, got, bias, w = _run(fmt, m, n, k, out_dtype, dev)
+    wt = torch.from_numpy(w).float()
+    _close(got, a.float() @ wt.T + bias, out_dtype, a, wt)
+
+
 # What the group kernel, which sums K in eight runs, is off the exact product by, and a tenth: 6.1e-8 of the norm, 8.0e-8
 # where scale2 rounds once more, 1.21e-7 for codes of one sign.
 RUN_ERROR = {"mxfp4": 6.7e-8, "nvfp4": 8.8e-8, "e4m3": 1.33e-7}
+
+
+# Workgroups are ceil(n / 256) x ceil(m / rows), and the tile is the largest that gives 256 of them: 64 rows at (40, ..) and
+# (1000, ..), 128 at the others in 4 bit (64 in 8 bit, which has no more).
+@pytest.mark.parametrize("fmt", ["mxfp4", "nvfp4", "fp8", "e4m3"])
+@pytest.mark.parametrize("m,n,k,out_dtype", [(40, 65550, 128, torch.bfloat16), (64, 65536, 128, torch.float32),
+                                             (70, 65550, 128, torch.bfloat16), (130, 33000, 256, torch.float32),
+                                             (1000, 4100, 256, torch.bfloat16), (2100, 4104, 256, torch.bfloat16)])
+def test_tiles_of_64_and_128_rows(dev, fmt, m, n, k, out_dtype):
+    print(f"{fmt} m={m} n={n} k={k} {out_dtype}", flush=True)
+    a, got, bias, w = _run(fmt, m, n, k, out_dtype, dev)
+    wt = torch.from_numpy(w).float()
+    _close(got, a.float() @ wt.T + bias, out_dtype, a, wt)
 
 
 # What the group kernel, which sums K in eight runs, is off the exact product by, and a tenth: 6.1e-8 of the norm, 8.0e-8
@@ -92,3 +119,24 @@ def test_layer_mlp_of_40_rows(dev, mlp_fmt):
                                        mlp_fmt=mlp_fmt)
     ref = olayer.gdn_layer_decode(x, w, st, cv, nk, nv, mlp_fmt=mlp_fmt)[0]
     torch.testing.assert_close(out.float().cpu(), ref.float(), **FUSED_TOL)
+
+
+@pytest.mark.parametrize("fmt,b", [("mxfp4", 1100), ("mxfp4", 2039), ("nvfp4", 1100), ("nvfp4", 2039), ("mxfp8", 1100)])
+def test_layer_tiles_of_64_and_128_rows(dev, fmt, b):
+    """A decode layer of hidden and MLP width 4096 and 2048 over 1100 (tiles of 64 rows) or 2039 sequences (128 in 4 bit):
+    the output projection, gate | up with SwiGLU, and down with the residual. The layer rounds to bf16 some ten times
+    (2^-9 each, about 6e-3 of a row's norm if all fell differently): every row and column within 2e-2 of its norm, where
+    16 wrong channels of a row are 6e-2."""
+    g = torch.Generator().manual_seed(b)
+    h, f, nk, nv = 4096, 2048, 1, 2
+    w = configs.gdn_layer_weights(g, h, f, nk, nv, proj_fmt=fmt, mlp_fmt=fmt)
+    x = torch.randn(b, h, generator=g).bfloat16()
+    st = torch.randn(b, nv, 128, 128, generator=g) * 0.02
+    cv = torch.randn(b, 3, 2 * nk * 128 + nv * 128, generator=g).bfloat16()
+    print(f"layer of {b} rows {fmt}", flush=True)
+    out, _, _ = layer.gdn_layer_decode(x.to(dev), {n: t.to(dev) for n, t in w.items()}, st.to(dev), cv.to(dev), nk, nv,
+                                       proj_fmt=fmt, mlp_fmt=fmt)
+    ref = olayer.gdn_layer_decode(x, w, st, cv, nk, nv, proj_fmt=fmt, mlp_fmt=fmt)[0].float()
+    d = out.float().cpu() - ref
+    for dim in (0, 1):
+        assert (d.norm(dim=dim) <= 2e-2 * ref.norm(dim=dim)).all(), float((d.norm(dim=dim) / ref.norm(dim=dim)).max())
