@@ -160,7 +160,7 @@ class MxLinearPrefillWorkload(Workload):
 
     name = "mxfp4_linear_prefill"
     tokens = 4096  # tokens one step carries through the path
-    kernel = "mx_gemm_kernel<0, 0>"
+    kernel = "mx_gemm_kernel<0, 0, 128, false>"
     timing = "graph"
     mfma = True
     traffic_profile = "mxfp4_linear_prefill_m4096_pmc.txt"

@@ -657,7 +657,9 @@ int axk_attn_layer_decode_moe(const uint16_t* x, const float* ln1, const uint8_t
  * result equals `tokens` successive decode-layer calls, one row each. Arguments otherwise as the decode layers.
  * ------------------------------------------------------------------------------------------- */
 
-/* Workspace bytes of axk_gdn_layer_verify / axk_attn_layer_verify (0 = unsupported shape; batch * tokens <= 4096). */
+/* Workspace bytes of axk_gdn_layer_verify / axk_attn_layer_verify (0 = unsupported shape; batch * tokens <= 4096). The
+ * attention layers' size ends with the KV-split scratch (axk_paged_prefill_workspace_size of the batch * tokens rows, to
+ * a multiple of 256); a workspace without it is accepted, and the attention then runs unsplit. */
 size_t axk_gdn_layer_verify_workspace_size(int64_t batch, int64_t tokens, int64_t hidden, int64_t num_k_heads,
                                            int64_t num_v_heads, int64_t head_dim, int64_t inter);
 size_t axk_attn_layer_verify_workspace_size(int64_t batch, int64_t tokens, int64_t hidden, int64_t num_qo_heads,
@@ -704,7 +706,8 @@ int axk_attn_layer_verify(const uint16_t* x, const float* ln1, const uint8_t* w_
  * per-row snapshots (the verify layers keep those). Arguments otherwise as the verify layers.
  * ------------------------------------------------------------------------------------------- */
 
-/* Workspace bytes of axk_gdn_layer_prefill / axk_attn_layer_prefill (0 = unsupported shape). */
+/* Workspace bytes of axk_gdn_layer_prefill / axk_attn_layer_prefill (0 = unsupported shape; the attention layer's as the
+ * verify layer's). */
 size_t axk_gdn_layer_prefill_workspace_size(int64_t batch, int64_t tokens, int64_t hidden, int64_t num_k_heads,
                                             int64_t num_v_heads, int64_t head_dim, int64_t inter);
 size_t axk_attn_layer_prefill_workspace_size(int64_t batch, int64_t tokens, int64_t hidden, int64_t num_qo_heads,
