@@ -1523,9 +1523,10 @@ __global__ __launch_bounds__(64 * kPfWaves, (D == 256 ? 1 : 2)) void paged_prefi
       tile_loads(ba, rows_of(na[j]), lds0 + j * C::PAIR);
       tile_loads(bb, rows_of(nb[j]), lds0 + j * C::PAIR + C::BUF);
     }
-    // the loop below takes pairs p_beg .. p_last - 1; at D <= 128 the last pair has code of its own (4096 tokens, HQ 8, HKV 2,
-    // D 128: 122 -> 114 us, a single pair 7.7 -> 6.7; at D = 256 that costs the loop 7 % of its time: 176 -> 189 us)
-    constexpr bool kPeel = D <= 128;
+    // the loop below takes pairs p_beg .. p_last - 1; at D = 128 the last pair has code of its own (4096 tokens, HQ 8, HKV 2:
+    // 122 -> 114 us, a single pair 7.7 -> 6.7). At D = 256 that costs the loop 7 % of its time (176 -> 189 us), at D = 64 the
+    // registers of a third wave a SIMD (41 x 3 tokens after 3589, 16 heads: 101 -> 121 us).
+    constexpr bool kPeel = D == 128;
     const int p_beg = t_beg / 2, p_last = (t_end + 1) / 2 - (kPeel ? 1 : 0);
     // the pair with tokens (a, b) in ring slot sl has landed for every wave: clear its tiles of pages outside the pool
     auto clear_bad = [&](int a, int b, int sl) {
