@@ -589,13 +589,15 @@ struct GateUpArgs {
 
 // gate-up + SwiGLU: workgroup (slot, ngrp-th run of kStreamWaves * tpw tiles); wave w streams tiles
 // run + w + kStreamWaves i.
-// STAGE (K a multiple of the batch's 128 kBatchChunks values): each batch's weights are loaded as whole row segments of
-// 64 kBatchChunks bytes (16 / kBatchChunks rows per load instruction, which keeps the address path's per-line work low),
-// written to a wave-private LDS tile and read back in the MFMA layout, and its E8M0 scales, 4 kBatchChunks consecutive
-// bytes of the row (chunks x lane groups), come with one load per matrix. Otherwise weights and scales are loaded unit by
-// unit. ROWS activation rows per pass.
-template <int ROWS, bool STAGE>
+// WIDE (K a multiple of the batch's 128 kBatchChunks values): a batch's E8M0 scales are 4 kBatchChunks
+// consecutive bytes of the row (chunks x lane groups), fetched with one load per matrix; otherwise one byte load
+// per unit.
+// STAGE (with WIDE): each batch's weights are loaded as whole row segments of 64 kBatchChunks bytes (16 / kBatchChunks
+// rows per load instruction, which keeps the address path's per-line work low), written to a wave-private LDS tile
+// and read back in the MFMA layout; ROWS activation rows per pass.
+template <bool WIDE, int ROWS, bool STAGE>
 __global__ __launch_bounds__(kStreamThreads) void moe_gateup_kernel(GateUpArgs a) {
+  static_assert(!STAGE || WIDE, "staged weights need whole batches");
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ SlotLds L;
   uint16_t* sA = reinterpret_cast<uint16_t*>(smem);
@@ -667,11 +669,13 @@ __global__ __launch_bounds__(kStreamThreads) void moe_gateup_kernel(GateUpArgs a
         const int64_t kb = min((int64_t)(bi * kBatchChunks + j) * 128 + 32 * g, (int64_t)H - 32);
         bt.qg[j] = load_nt(past ? idle + 32 * j : gw + n * (H / 2) + kb / 2);
         bt.qu[j] = load_nt(past ? idle + 32 * j + 16 : uw + n * (H / 2) + kb / 2);
-        bt.sg[j] = gs[n * (H / 32) + kb / 32];
-        bt.su[j] = us[n * (H / 32) + kb / 32];
+        if (!WIDE) {
+          bt.sg[j] = gs[n * (H / 32) + kb / 32];
+          bt.su[j] = us[n * (H / 32) + kb / 32];
+        }
       }
     }
-    if (STAGE) {
+    if (WIDE) {
       load_scale_words(bt.sg, gs + n * (H / 32) + 4 * kBatchChunks * bi);
       load_scale_words(bt.su, us + n * (H / 32) + 4 * kBatchChunks * bi);
     }
@@ -705,12 +709,12 @@ __global__ __launch_bounds__(kStreamThreads) void moe_gateup_kernel(GateUpArgs a
 #pragma unroll
       for (int j = 0; j < kBatchChunks; ++j) {
         const int c = bi * kBatchChunks + j;
-        if (!STAGE && c * 128 >= H) continue;  // whole chunk past K (uniform)
+        if (!WIDE && c * 128 >= H) continue;  // whole chunk past K (uniform)
         const int kb = c * 128 + 32 * g;
-        const bool kv = STAGE || kb < H;       // this lane's unit (a chunk can straddle the end of K)
+        const bool kv = WIDE || kb < H;       // this lane's unit (a chunk can straddle the end of K)
         const int kc = kv ? kb : H - 32;
-        const uint32_t bg = STAGE ? (cur.sg[j] >> (8 * g)) & 0xffu : cur.sg[j];
-        const uint32_t bu = STAGE ? (cur.su[j] >> (8 * g)) & 0xffu : cur.su[j];
+        const uint32_t bg = WIDE ? (cur.sg[j] >> (8 * g)) & 0xffu : cur.sg[j];
+        const uint32_t bu = WIDE ? (cur.su[j] >> (8 * g)) & 0xffu : cur.su[j];
         const float scg = kv ? e8m0_to_f32(bg) : 0.f, scu = kv ? e8m0_to_f32(bu) : 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -774,8 +778,9 @@ struct DownArgs {
 };
 
 // down: workgroup (slot, run of kStreamWaves * tpw 16-row tiles of H); routed rows scaled by their routing weight.
-template <int ROWS, bool STAGE>
+template <bool WIDE, int ROWS, bool STAGE>
 __global__ __launch_bounds__(kStreamThreads) void moe_down_kernel(DownArgs a) {
+  static_assert(!STAGE || WIDE, "staged weights need whole batches");
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ SlotLds L;
   uint16_t* sA = reinterpret_cast<uint16_t*>(smem);
@@ -839,10 +844,10 @@ __global__ __launch_bounds__(kStreamThreads) void moe_down_kernel(DownArgs a) {
       for (int j = 0; j < kBatchChunks; ++j) {
         const int64_t kb = min((int64_t)(bi * kBatchChunks + j) * 128 + 32 * g, (int64_t)K - 32);
         bt.q[j] = load_nt(past ? idle + 16 * j : dw + n * (K / 2) + kb / 2);
-        bt.s[j] = ds[n * (K / 32) + kb / 32];
+        if (!WIDE) bt.s[j] = ds[n * (K / 32) + kb / 32];
       }
     }
-    if (STAGE) load_scale_words(bt.s, ds + n * (K / 32) + 4 * kBatchChunks * bi);
+    if (WIDE) load_scale_words(bt.s, ds + n * (K / 32) + 4 * kBatchChunks * bi);
   };
 
   int m0 = mbeg;
@@ -887,11 +892,11 @@ __global__ __launch_bounds__(kStreamThreads) void moe_down_kernel(DownArgs a) {
 #pragma unroll
       for (int j = 0; j < kBatchChunks; ++j) {
         const int c = bi * kBatchChunks + j;
-        if (!STAGE && c * 128 >= K) continue;
+        if (!WIDE && c * 128 >= K) continue;
         const int kb = c * 128 + 32 * g;
-        const bool kv = STAGE || kb < K;
+        const bool kv = WIDE || kb < K;
         const int kc = kv ? kb : K - 32;
-        const uint32_t sb = STAGE ? (cur.s[j] >> (8 * g)) & 0xffu : cur.s[j];
+        const uint32_t sb = WIDE ? (cur.s[j] >> (8 * g)) & 0xffu : cur.s[j];
         const float sc = kv ? e8m0_to_f32(sb) : 0.f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -1585,21 +1590,26 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   const int max_slots = E < T * K ? E : T * K;
   const int fmax = F > Fs ? F : Fs;
   // runs of 4 x tpw tiles per workgroup; activation rows staged in dynamic LDS ([rows][K + 8] bf16). Where K is a
-  // multiple of 256 the weights are staged through LDS as whole row segments, with 8, 12 or 16 activation rows per pass
-  // by how many rows an expert has on average (T K / E); the others stream MFMA-layout units with 16 rows per pass.
+  // multiple of 256 and an expert has few rows on average (T K / E), the weights are staged through LDS as whole row
+  // segments, with 8, 12 or 16 activation rows per pass; the others stream MFMA-layout units with 16 rows per pass, since
+  // each further pass streams the expert's weights again.
   // Measured (E 256, top-8, H 2048, F 512; us at 65 / 100 / 150 / 200 / 256 tokens): unstaged 16 rows above 64 tokens
   // 120 / 133 / 155 / 161 / 173; staged, gate-up 8 rows and down 8 99 / 114 / 138 / 163 / 189, gate-up 8 and down 16 102 / 114 /
-  // 138 / 155 / 173, gate-up 12 and down 16 112 / 122 / 142 / 150 / 166.
+  // 138 / 155 / 173, gate-up 12 and down 16 112 / 122 / 142 / 150 / 166. From 8 rows an expert on unstaged is the faster
+  // (E 128, top-8, H 4096, F 1536, 100 / 160 / 256 tokens: 428 / 486 / 738 us, staged 411 / 501 / 785; E 8, top-2, H and F
+  // 4096, 65 / 160 / 256: 207 / 398 / 594, staged 220 / 445 / 656).
   const int gu_tpw = kGateUpTilesPerWave, dn_tpw = kDownTilesPerWave;
   const int run_gu = kStreamWaves * gu_tpw, run_dn = kStreamWaves * dn_tpw;
   const int gu_grp = ((fmax + 15) / 16 + run_gu - 1) / run_gu;
   const int dn_grp = ((H + 15) / 16 + run_dn - 1) / run_dn;
-  const int batch_k = 128 * kBatchChunks;
+  const int wide_k = 128 * kBatchChunks;
+  const bool gu_wide = H % wide_k == 0, dn_wide = F % wide_k == 0 && Fs % wide_k == 0;
   const size_t stage_lds = kStreamWaves * kWaveStageBytes;
   const bool many = T > 64;  // (a size that 16 unstaged rows would not fit is refused there, staged or not)
   AXK_REQUIRE(!many || (stream_stage_off(kStageRows, H) <= kMaxStreamLds &&
                         stream_stage_off(kStageRows, fmax) <= kMaxStreamLds), AXK_E_SHAPE);
-  const bool gu_stage = H % batch_k == 0, dn_stage = F % batch_k == 0 && Fs % batch_k == 0;
+  const bool few = !many || (int64_t)T * K <= 8 * (int64_t)E;
+  const bool gu_stage = gu_wide && few, dn_stage = dn_wide && few;
   const bool gu_mid = gu_stage && many && (int64_t)T * K > 5 * (int64_t)E &&
                       stream_stage_off(kMidRows, H) + stage_lds <= kMaxStreamLds;
   const bool dn_full = dn_stage && many && (int64_t)T * K > 4 * (int64_t)E &&
@@ -1611,12 +1621,14 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   AXK_REQUIRE(gu_lds <= kMaxStreamLds && dn_lds <= kMaxStreamLds, AXK_E_SHAPE);
   static AxkOnce lds_once;  // > 64 KiB of dynamic LDS must be allowed once per kernel
   const int raised = axk_once(lds_once, [] {
-    const void* fns[6] = {reinterpret_cast<const void*>(&moe_gateup_kernel<kMidRows, true>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<kStageRows, true>),
-                          reinterpret_cast<const void*>(&moe_gateup_kernel<kStageRows, false>),
-                          reinterpret_cast<const void*>(&moe_gateup_kernel<kSmallRows, true>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<kStageRows, false>),
-                          reinterpret_cast<const void*>(&moe_down_kernel<kSmallRows, true>)};
+    const void* fns[8] = {reinterpret_cast<const void*>(&moe_gateup_kernel<true, kMidRows, true>),
+                          reinterpret_cast<const void*>(&moe_gateup_kernel<true, kStageRows, false>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<true, kStageRows, true>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<true, kStageRows, false>),
+                          reinterpret_cast<const void*>(&moe_gateup_kernel<false, kStageRows, false>),
+                          reinterpret_cast<const void*>(&moe_gateup_kernel<true, kSmallRows, true>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<false, kStageRows, false>),
+                          reinterpret_cast<const void*>(&moe_down_kernel<true, kSmallRows, true>)};
     for (const void* f : fns) {
       const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxStreamLds);
       if (e != hipSuccess) return e;
@@ -1629,18 +1641,22 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
                 gu_nsp, w};
   const dim3 gu_grid((unsigned)((max_slots + gu_nsp) * gu_grp)), dn_grid((unsigned)((max_slots + dn_nsp) * dn_grp));
   if (gu_mid)
-    hipLaunchKernelGGL((moe_gateup_kernel<kMidRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+    hipLaunchKernelGGL((moe_gateup_kernel<true, kMidRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   else if (gu_stage)
-    hipLaunchKernelGGL((moe_gateup_kernel<kSmallRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+    hipLaunchKernelGGL((moe_gateup_kernel<true, kSmallRows, true>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+  else if (gu_wide)
+    hipLaunchKernelGGL((moe_gateup_kernel<true, kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   else
-    hipLaunchKernelGGL((moe_gateup_kernel<kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
+    hipLaunchKernelGGL((moe_gateup_kernel<false, kStageRows, false>), gu_grid, dim3(64 * kStreamWaves), gu_lds, st, ga);
   DownArgs da{e_dw, e_ds, sh_down_w, sh_down_s, topk_ids, topk_weights, T, H, F, Fs, E, K, dn_grp, dn_tpw, dn_nsp, w};
   if (dn_full)
-    hipLaunchKernelGGL((moe_down_kernel<kStageRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+    hipLaunchKernelGGL((moe_down_kernel<true, kStageRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   else if (dn_stage)
-    hipLaunchKernelGGL((moe_down_kernel<kSmallRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+    hipLaunchKernelGGL((moe_down_kernel<true, kSmallRows, true>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+  else if (dn_wide)
+    hipLaunchKernelGGL((moe_down_kernel<true, kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   else
-    hipLaunchKernelGGL((moe_down_kernel<kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
+    hipLaunchKernelGGL((moe_down_kernel<false, kStageRows, false>), dn_grid, dim3(64 * kStreamWaves), dn_lds, st, da);
   // the decode router formed the shared gate's logit when the routing ran in this call (gate_given)
   CombineArgs ca{h2, x_res, w_shg, gate_given ? w.gate_logit : nullptr, topk_ids, combine_shared, T, H, E, K, w, out};
   launch_combine<false>(ca, st);
