@@ -59,17 +59,28 @@ constexpr int64_t kMaxPrefillTokens = 1 << 16;
 constexpr int64_t kMaxPrefillPairs = 1 << 19;
 constexpr int kBlkTokens = 256;  // tokens per block of the prefill grouping
 constexpr int kBM = 128, kBK = 64;  // prefill GEMM: rows of a tile where experts have many, K step
-// The rows of a tile: 32 or 64 where the experts' rows are few on average (T K / E), so that the GEMMs neither load nor
-// multiply tiles that are mostly padding. Measured (E 256, top-8, H 2048, F 512; us with 32- / 64- / 128-row tiles):
-// 257 tokens 182 / 193 / 216, 700 tokens 196 / 206 / 227, 1024 tokens 227 / 216 / 236, 1400 tokens 266 / 227 / 246,
-// 2048 tokens 320 / 273 / 272, 4096 tokens 544 / 428 / 408. Around 128 rows an expert, half the experts have a few more
-// than a 128-row tile takes, and their second tiles stream and decode the weights again: 160-row tiles there (4096
-// tokens 426 -> 397 us on one box; 2800 tokens, whose experts fit 128 rows, 328 -> 348). At the band's edges: 3850 tokens
-// (120.3 rows an expert) 379 us, 3840 in 128 rows 381; 5280 (165) 515, 5300 in 128 rows 518.
+// The rows of a tile, by the rows an expert has on average (T K / E). 32 or 64 where these are few, so that the GEMMs
+// neither load nor multiply tiles that are mostly padding, and 160 a little above 128, where half the experts have a few
+// more rows than a 128-row tile takes, and their second tiles stream and decode the weights again. Measured, us with 32- /
+// 64- / 128- / 160-row tiles at the average rows given:
+//   E 256, top-8, H 2048, F 512:  24: 197 / 205 / 226 / 247, 32: 229 / 213 / 234 / 255, 56: 290 / 244 / 254 / 275, 72: 358 / 300 / 288 / 309,
+//                                 122: 531 / 408 / 387 / 381, 144: 607 / 477 / 476 / 441, 160: 659 / 514 / 507 / 504
+//   E 256, top-8, H 7168, F 512:  24: 695 / 760 / 764 / 934, 32: 827 / 783 / 790 / 976, 44: 979 / 841 / 840 / 1069,
+//                                 56: 1097 / 935 / 901 / 1163, 128: 2088 / 1552 / 1420 / 1631, 144: 2316 / 1749 / 1626 / 1572,
+//                                 160: 2520 / 1864 / 1721 / 1731
+//   E 128, top-8, H 4096, F 1536: 24: 610 / 622 / 576 / 654, 44: 820 / 671 / 616 / 719, 128: 1646 / 1125 / 989 / 1043, 144: 1822 / 1289 / 1184 / 1072
+//   E 64, top-6, H 2048, F 1408:  44: 205 / 176 / 174 / 190, 122: 355 / 264 / 257 / 254, 144: 398 / 302 / 296 / 271
+//   E 32, top-4, H and F 2880:    44: 332 / 243 / 332 / 373, 56: 349 / 272 / 338 / 386, 128: 580 / 446 / 470 / 448, 144: 641 / 488 / 557 / 468
+// So with a long down reduction (F above 1024) the smaller tiles gain nothing, but for the 64-row tile where H leaves no
+// whole scale dwords and the 128-row tile's scale tables cost it more than its rows give; and from H 4096 on, where the
+// weights of an expert are long streams, the 64-row tile ends earlier and the 160-row tile's band is narrower.
 constexpr int kBMWide = 160;
-inline int tile_rows(int64_t T, int64_t E, int64_t K) {
+inline int tile_rows(int64_t T, int64_t E, int64_t K, int64_t H, int64_t F) {
   const int64_t p = T * K;
-  return p <= 26 * E ? 32 : p <= 56 * E ? 64 : p > 120 * E && p <= 165 * E ? kBMWide : kBM;
+  const bool dwords = H % 128 == 0;
+  if (p <= 26 * E && F <= 1024 && dwords) return 32;
+  if (p <= (H >= 4096 ? 40 : 56) * E && (F <= 1024 || !dwords)) return 64;
+  return p > (H >= 4096 ? 136 : 120) * E && p <= (H >= 4096 ? 152 : 165) * E ? kBMWide : kBM;
 }
 
 struct MoeWs {
@@ -95,8 +106,7 @@ struct MoeWs {
 };
 
 int64_t prefill_blocks(int64_t T) { return (T + kBlkTokens - 1) / kBlkTokens; }
-int64_t prefill_max_tiles(int64_t T, int64_t E, int64_t K) {
-  const int64_t tb = tile_rows(T, E, K);
+int64_t prefill_max_tiles(int64_t T, int64_t E, int64_t K, int64_t tb) {
   return (T * K + tb - 1) / tb + E + (T + tb - 1) / tb;
 }
 
@@ -138,7 +148,7 @@ MoeWs moe_ws(void* ws, int64_t T, int64_t H, int64_t E, int64_t K, int64_t F, in
   unsigned char* b = reinterpret_cast<unsigned char*>(ws);
   // a list of 32- or 64-row tiles, longer than its part, takes the half of y that bf16 rows leave (2 T K H bytes, H at
   // least 64; the list at most T K / 2 + 16 E + T / 2 + 48, E at most 1024)
-  const size_t tiles = T > kDecodeTokens && tile_rows(T, E, K) < kBM ? off[9] + (size_t)T * K * H * 2 : off[12];
+  const size_t tiles = T > kDecodeTokens && tile_rows(T, E, K, H, F) < kBM ? off[9] + (size_t)T * K * H * 2 : off[12];
   return {reinterpret_cast<int*>(b + off[0]),       reinterpret_cast<int*>(b + off[1]),
           reinterpret_cast<int4*>(b + off[2]),      reinterpret_cast<int*>(b + off[3]),
           reinterpret_cast<int*>(b + off[4]),       reinterpret_cast<int*>(b + off[5]),
@@ -1558,12 +1568,12 @@ int moe_experts_impl(const uint16_t* h2, const uint16_t* x_res, const uint16_t* 
   const int combine_shared = (has_shared || y_sh_given) ? 1 : 0;
   const int T = (int)tokens, H = (int)hidden, E = (int)num_experts, K = (int)top_k, F = (int)inter, Fs = (int)d.Fs;
   if (T > kDecodeTokens) {
-    const int NB = (int)prefill_blocks(T), tb = tile_rows(T, E, K);
+    const int NB = (int)prefill_blocks(T), tb = tile_rows(T, E, K, H, F);
     // the (block, expert) counts: counted by the routing launch when it ran in this call, else from the ids
     if (!counted) hipLaunchKernelGGL(moe_pcount_kernel, dim3((unsigned)NB), dim3(256), 0, st, topk_ids, T, E, K, w);
     hipLaunchKernelGGL(moe_pscan_kernel, dim3(1), dim3(256), 0, st, T, E, NB, has_shared ? 1 : 0, tb, w);
     hipLaunchKernelGGL(moe_pscatter_kernel, dim3((unsigned)NB), dim3(256), 0, st, topk_ids, topk_weights, T, E, K, w);
-    const unsigned tiles = (unsigned)prefill_max_tiles(T, E, K);
+    const unsigned tiles = (unsigned)prefill_max_tiles(T, E, K, tb);
     const int fmax = F > Fs ? F : Fs;
     GGemmArgs gu{h2, nullptr, e_gw, e_gs, sh_gate_w, sh_gate_s, sh_up_w, sh_up_s, T, H, F, Fs, fmax, w};
     // per-step scale dwords (SDMA) where every scale row of the reduction is whole, aligned dwords
